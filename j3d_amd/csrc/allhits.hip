@@ -111,8 +111,9 @@ __device__ inline uint32_t vox_color_index(uint32_t r, uint32_t g, uint32_t b) {
 template <int W>
 __global__ void __launch_bounds__(kAllBlock) k_all_hits(AllHitsArgs a) {
   extern __shared__ uint2 lds_stack[];
-  Stack<kAllD> st;
-  st.init(lds_stack, a.spill, a.spill_cap);
+  StackArea area;
+  area.init(lds_stack, a.spill, a.spill_cap);
+  Stack<kAllD> st(area);
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= a.n) return;
   const bool vox = a.rays == nullptr;

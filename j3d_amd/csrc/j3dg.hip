@@ -190,14 +190,16 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
   // on every ray start and hit completion: keep the block's copy in LDS
   constexpr bool kLdsObjects = M != kModeBatch && !kTop;
   __shared__ DevObject s_objs[kLdsObjects ? J3DG_MAX_OBJECTS : 1];
+  __shared__ uint32_t s_drained;  // the work bands that this block's waves found drained
+  if (threadIdx.x == 0) s_drained = 0;
   if (kLdsObjects) {
     n_obj = min(n_obj, (uint32_t)J3DG_MAX_OBJECTS);
     const uint32_t words = n_obj * (uint32_t)(sizeof(DevObject) / 4);
     const uint32_t* src = reinterpret_cast<const uint32_t*>(objs);
     uint32_t* dst = reinterpret_cast<uint32_t*>(s_objs);
     for (uint32_t i = threadIdx.x; i < words; i += blockDim.x) dst[i] = gload(src + i);
-    __syncthreads();
   }
+  __syncthreads();
   const DevObject* const tab = kLdsObjects ? s_objs : objs;
   const TopNode* const top = kTop ? static_cast<const TopNode*>(f.top_nodes) : nullptr;
   // a small top level is copied into LDS after the stack (all threads reach the barrier)
@@ -210,8 +212,9 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
     __syncthreads();
     top_l = (lds_top*)(lds_stack + D * blockDim.x);
   }
-  Stack<D> st;
-  st.init(lds_stack, spill, spill_cap);
+  StackArea area;
+  area.init(lds_stack, spill, spill_cap);
+  Stack<D> st(area);
   Counters c = {0, 0, 0}, cs = {0, 0, 0};  // primary (or query) / shadow-phase work
   uint32_t acc[6] = {0, 0, 0, 0, 0, 0};  // wave-uniform event counts
   uint32_t trips = 0;
@@ -225,7 +228,7 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
   uint64_t tl_start = COUNT ? (uint64_t)wall_clock64() : 0, tl_exh = 0, tl_coop = 0;
   uint32_t trips_coop = 0;
   RayPool pool;
-  pool.init();
+  pool.init(&s_drained);
   uint32_t n_rays = n_rays_q;
   if (kIsFrame) n_rays = f.n_tiles * 64u;
   if (M == kModeShadow) n_rays = __builtin_amdgcn_readfirstlane(*q.count);
@@ -290,13 +293,14 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
     shfl_from(wd, src);
     shfl_from(s, src);
     shfl_from(best, src);
-    shfl_from(st, src);
+    shfl_from(st.col, src);
+    shfl_from(st.sp, src);
   };
   // split mode: a lane that starts idle, with an empty stack in the column of
   // the k-th lane of `free_cols` (lanes of this wave whose columns nobody owns)
   auto fresh_helper = [&](uint64_t free_cols, uint32_t k) {
     for (uint32_t i = 0; i < k; ++i) free_cols &= free_cols - 1u;
-    st.init(lds_stack, spill, spill_cap, (threadIdx.x & ~63u) + (uint32_t)__builtin_ctzll(free_cols));
+    st.reset((threadIdx.x & ~63u) + (uint32_t)__builtin_ctzll(free_cols));
     s.cur = kNone;
   };
 
@@ -307,8 +311,7 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
     if (!pool.exhausted && (n_idle >= refill_min || n_idle == 64)) {
       // hand new rays to idle lanes; ids outside the rectangle leave a lane idle, so repeat
       while (__ballot(phase == 0) && !pool.exhausted) {
-        uint32_t id = kIsFrame ? pool.take_banded(phase == 0, queue, batch, f.n_tiles)
-                                         : pool.take(phase == 0, queue, batch, n_rays);
+        const uint32_t id = pool.take(phase == 0, queue, batch, n_rays, kIsFrame && f.pixel_cost ? kBandBlock : 1u);
         if (id == kNone) continue;
         float tn, tf;
         if (kFrameLike) {
@@ -420,7 +423,7 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
       const uint32_t n = (uint32_t)__popcll(heads);
       const uint32_t ng = n <= 8u ? 8u : n <= 16u ? 4u : 2u;
       if (n > 0u && ng > gsz) {
-        const uint32_t col = (uint32_t)(st.lds - (lds_entry*)lds_stack) & 63u;
+        const uint32_t col = st.col & 63u;
         uint64_t used = 0;
         for (uint32_t b = 0; b < 64u; ++b)
           if (__ballot(phase != 0u && col == b)) used |= 1ull << b;
@@ -447,13 +450,14 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
       bool done;
       if (lnobj == 0 || (kTop && phase != kFinishPhase && s.cur == kNone)) {
         done = true;  // no object, or (top level) no object box on the ray's way or a ray that is not finite
-      } else if (kFrameLike && (phase == kFinishPhase || (W == 8 && !coop))) {
+      } else if ((kFrameLike && phase == kFinishPhase) || (W == 8 && !coop)) {
         // one fetch for every lane: a node, a leaf's triangles or a hit's completion record
-        const float4* p = phase == kFinishPhase ? lobjs[best.obj].fin + 3 * (size_t)best.tri : step_fetch(s);
+        const bool fin = kFrameLike && phase == kFinishPhase;
+        const float4* p = fin ? lobjs[best.obj].fin + 3 * (size_t)best.tri : step_fetch(s);
         float4 v[6];
 #pragma unroll
         for (int k = 0; k < 6; ++k) v[k] = gload4(p + k);
-        if (phase == kFinishPhase) {
+        if (fin) {
           done = false;
           phase = 0;
           const FrameParams& F = frame_ref<M>(f, bp, fi);

@@ -101,62 +101,76 @@ __device__ inline Ray make_object_ray(const float* inv_cs, f4 o, f4 d, float tn,
 // serialise every push and pop against the lane's outstanding loads and stores.
 typedef uint32_t j3d_u32x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(3))) j3d_u32x2 lds_entry;
+typedef __attribute__((address_space(3))) uint32_t lds_word;
 typedef __attribute__((address_space(1))) j3d_u32x2 glb_entry;
+
+// What every lane's stack of a launch shares (wave-uniform: kept out of the
+// lane state, so that it stays in scalar registers when the tail modes move a
+// ray between lanes).
+struct StackArea {
+  lds_entry* lds;    // entry 0 of the block's column 0
+  glb_entry* spill;  // spill area of the grid: [entry][lane]
+  uint64_t sstride;  // lanes of the grid
+  uint32_t cap;      // spill entries per lane
+  uint32_t shift;    // log2(threads per block): an LDS entry row holds one entry of every thread
+  __device__ void init(uint2* lds_base, uint2* spill_base, uint32_t spill_cap) {
+    lds = (lds_entry*)lds_base;
+    spill = (glb_entry*)spill_base + (uint64_t)blockIdx.x * blockDim.x;
+    sstride = (uint64_t)gridDim.x * blockDim.x;
+    cap = spill_cap;
+    shift = 31u - (uint32_t)__clz(blockDim.x);  // blocks are 64, 128 or 256 threads
+  }
+};
 
 template <int D>
 struct Stack {
-  lds_entry* lds;    // &lds[0][tid], stride `stride`
-  uint32_t stride;   // threads per block
-  glb_entry* spill;  // &spill[0][global lane]
-  uint64_t sstride;  // lanes of the grid
-  uint32_t cap;      // spill entries per lane
+  const StackArea& a;
+  uint32_t col;  // the thread of the block whose LDS and spill columns hold this stack
   uint32_t sp;
   bool overflow;
 
-  __device__ void init(uint2* lds_base, uint2* spill_base, uint32_t spill_cap) {
-    init(lds_base, spill_base, spill_cap, threadIdx.x);
-  }
-  // an empty stack in the LDS and spill column of thread `col` of the block
-  __device__ void init(uint2* lds_base, uint2* spill_base, uint32_t spill_cap, uint32_t col) {
-    lds = (lds_entry*)lds_base + col;
-    stride = blockDim.x;
-    sstride = (uint64_t)gridDim.x * blockDim.x;
-    spill = (glb_entry*)spill_base + ((uint64_t)blockIdx.x * blockDim.x + col);
-    cap = spill_cap;
+  __device__ explicit Stack(const StackArea& area) : a(area), overflow(false) { reset(threadIdx.x); }
+  // an empty stack in the LDS and spill column of thread `column` of the block
+  __device__ void reset(uint32_t column) {
+    col = column;
     sp = 0;
-    overflow = false;
+  }
+  // LDS place of entry e (0-based from the bottom)
+  __device__ lds_entry* slot(uint32_t e) const { return a.lds + (((e & (D - 1)) << a.shift) + col); }
+  // spill place of entry e (after D newer entries)
+  __device__ glb_entry* spilled(uint32_t e) const { return a.spill + ((uint64_t)e * a.sstride + col); }
+  // entry e - D makes room for entry e >= D; false when the spill column is full
+  // (its size comes from the builder's stack bound; never expected)
+  __device__ bool move_out(uint32_t e) {
+    if (e - D >= a.cap) {
+      overflow = true;
+      return false;
+    }
+    *spilled(e - D) = *slot(e);
+    return true;
   }
   // stores entry e (0-based from the bottom) of this lane; false on overflow
   __device__ bool put(uint32_t e, uint32_t ref, float dist) {
-    const uint32_t slot = e & (D - 1);
-    if (e >= (uint32_t)D) {
-      if (e - D >= cap) {  // cap comes from the builder's stack bound; never expected
-        overflow = true;
-        return false;
-      }
-      spill[(uint64_t)(e - D) * sstride] = lds[slot * stride];
-    }
+    const bool room = e < (uint32_t)D || move_out(e);
     // lanes sharing one stack (the cooperative tail) all read the slot for
     // the spill before any of them overwrites it; see pop
     __builtin_amdgcn_wave_barrier();
-    j3d_u32x2 v = {ref, __float_as_uint(dist)};
-    lds[slot * stride] = v;
-    return true;
+    const j3d_u32x2 v = {ref, __float_as_uint(dist)};
+    *slot(e) = v;
+    return room;
   }
-  __device__ void push(uint32_t ref, float dist) {
-    if (put(sp, ref, dist)) ++sp;
-  }
+  __device__ void push(uint32_t ref, float dist) { sp += put(sp, ref, dist) ? 1u : 0u; }
   __device__ bool pop(uint32_t& ref, float& dist) {
     if (sp == 0) return false;
     --sp;
-    const uint32_t slot = sp & (D - 1);
-    const j3d_u32x2 v = lds[slot * stride];
+    lds_entry* const at = slot(sp);
+    const j3d_u32x2 v = *at;
     // In the cooperative tail the lanes of a group pop one shared stack: each
     // reads the top entry before any of them writes the spilled entry below it
     // back into that slot.  The wave executes both in lockstep; the barrier
     // (no instruction) keeps the compiler from moving the write above the read.
     __builtin_amdgcn_wave_barrier();
-    if (sp >= (uint32_t)D) lds[slot * stride] = spill[(uint64_t)(sp - D) * sstride];
+    if (sp >= (uint32_t)D) *at = *spilled(sp - D);
     ref = v.x;
     dist = __uint_as_float(v.y);
     return true;
@@ -463,12 +477,17 @@ __device__ inline uint32_t rank_in_mask(uint64_t m) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
-// Frames split their tile sequence into kBands bands of consecutive
-// kBandBlock-tile blocks, one per XCD: workgroups are dispatched to the eight
-// XCDs round robin, so block b starts on band b % 8, and each XCD's L2
-// serves the rays of one compact image band.  A wave whose band is drained
-// moves on to the next band.  Each band has its own queue counter, 64 bytes
-// apart, from word kBandQueue of the queue array.
+// Launches split their sequence of tiles (64 rays) into kBands bands of
+// consecutive tiles, one per XCD: workgroups are dispatched to the eight XCDs
+// round robin, so block b starts on band b % 8, and each XCD's L2 serves the
+// rays of one compact image band.  A wave whose band is drained moves on to
+// another one.  Each band has its own queue counter, 64 bytes apart, from word
+// kBandQueue of the queue array: one address takes an atomic every ~13 ns,
+// whoever asks, so a launch of many tiles must not draw them from one counter
+// (a batch of 24 frames, 316,000 tiles: 4.08 ms with one counter, one tile per
+// atomic; 2.44 ms with the bands and share()).  Frames in cost order cut their
+// bands at multiples of kBandBlock tiles (the order is sorted within bands),
+// other launches at any tile.
 constexpr uint32_t kXcds = 8;
 constexpr uint32_t kBandsPerXcd = 1;  // 2 and 4 (an XCD draining its bands in turn) measured slower
 constexpr uint32_t kBands = kXcds * kBandsPerXcd;
@@ -476,10 +495,11 @@ constexpr uint32_t kBandBlock = 256;
 constexpr uint32_t kBandQueue = 32;
 constexpr uint32_t kQueueWords = kBandQueue + 16 * kBands;
 
-// First ray id (tile position * 64) of band b of a frame of n_tiles tiles.
-__host__ __device__ inline uint32_t band_first_ray(uint32_t b, uint32_t n_tiles) {
-  const uint32_t nb = (n_tiles + kBandBlock - 1) / kBandBlock;
-  const uint32_t t = (b * nb / kBands) * kBandBlock;
+// First ray id (tile position * 64) of band b of n_tiles tiles, bands being
+// cut at multiples of `unit` tiles.
+__host__ __device__ inline uint32_t band_first_ray(uint32_t b, uint32_t n_tiles, uint32_t unit) {
+  const uint32_t nb = (n_tiles + unit - 1) / unit;
+  const uint32_t t = (uint32_t)((uint64_t)b * nb / kBands) * unit;
   return (t < n_tiles ? t : n_tiles) * 64u;
 }
 
@@ -487,66 +507,69 @@ __host__ __device__ inline uint32_t band_first_ray(uint32_t b, uint32_t n_tiles)
 struct RayPool {
   uint32_t next, end;
   bool exhausted;
-  uint32_t band, tried;  // banded frames: current band, bands drained so far
-  __device__ void init() {
+  uint32_t band;
+  uint32_t items;  // work items the next atomic takes; 0 on coming to a band
+  lds_word* drained;  // mask of the bands a wave of this block has seen drained
+  __device__ void init(uint32_t* block_drained) {
     next = end = 0;
     exhausted = false;
     band = (blockIdx.x % kXcds) * kBandsPerXcd;
-    tried = 0;
+    items = 0;
+    drained = (lds_word*)block_drained;
   }
-  // Refills [next, end) from the frame's bands (all lanes must call).
-  __device__ void refill_banded(uint32_t* queue, uint32_t batch, uint32_t n_tiles) {
-    while (tried < kBands) {
-      const uint32_t lo = band_first_ray(band, n_tiles), hi = band_first_ray(band + 1, n_tiles);
-      uint32_t base = 0;
-      if (lane_id() == 0) base = atomicAdd(queue + kBandQueue + 16 * band, batch);
-      base = __builtin_amdgcn_readfirstlane(__shfl(base, 0, 64));
-      if (base < hi - lo) {
+  // Work items to take at once with `left` rays left in the band: two while
+  // every wave can still take sixteen, which halves the atomics of a long
+  // queue.  Longer runs lose more to the uneven work of neighbouring tiles
+  // than they save (24 frames, 316,000 tiles: 2.44 ms with at most 2 items,
+  // 2.59, 2.86 and 3.58 ms with 4, 8 and 32), and frames in cost order, whose
+  // heaviest tiles are neighbours, take one at a time (28M-triangle 1080p
+  // frame: 0.74 ms with one, 0.87 ms with two).
+  __device__ static uint32_t share(uint32_t left, uint32_t batch, uint32_t unit) {
+    const uint32_t waves = (gridDim.x * (blockDim.x >> 6) + kBands - 1u) / kBands;
+    return unit == 1u && left / (16u * batch) >= waves ? 2u : 1u;
+  }
+  // Refills [next, end) from the bands (all lanes must call).
+  __device__ void refill(uint32_t* queue, uint32_t batch, uint32_t n_rays, uint32_t unit) {
+    const uint32_t n_tiles = (n_rays + 63u) >> 6;
+    for (;;) {
+      // skip the bands that waves of this block found drained: a failing atomic
+      // costs as much as one that brings work, and every wave would make eight
+      const uint32_t gone = __builtin_amdgcn_readfirstlane(*(volatile lds_word*)drained);
+      if (gone == (1u << kBands) - 1u) break;
+      while (gone >> band & 1u) {
+        band = band + 1 == kBands ? 0 : band + 1;
+        items = 0;
+      }
+      const uint32_t lo = band_first_ray(band, n_tiles, unit);
+      const uint32_t hi = min(band_first_ray(band + 1, n_tiles, unit), n_rays);
+      const uint32_t size = hi > lo ? hi - lo : 0u;
+      if (items == 0) items = share(size, batch, unit);
+      const uint32_t amount = items * batch;
+      uint32_t base = size;
+      if (size) {
+        if (lane_id() == 0) base = atomicAdd(queue + kBandQueue + 16 * band, amount);
+        base = __builtin_amdgcn_readfirstlane(__shfl(base, 0, 64));
+      }
+      if (base < size) {
         next = lo + base;
-        end = min(next + batch, hi);
+        end = hi - next > amount ? next + amount : hi;
+        items = share(size - base, batch, unit);
         return;
       }
-      band = band + 1 == kBands ? 0 : band + 1;
-      ++tried;
+      if (lane_id() == 0) atomicOr((uint32_t*)drained, 1u << band);
+      __builtin_amdgcn_wave_barrier();
     }
     exhausted = true;
   }
-  // As take, for a frame's banded tile sequence.
-  __device__ uint32_t take_banded(bool want, uint32_t* queue, uint32_t batch, uint32_t n_tiles) {
-    uint32_t id = kNone;
-    uint64_t m = __ballot(want);
-    while (m && !exhausted) {
-      if (next >= end) {
-        refill_banded(queue, batch, n_tiles);
-        if (exhausted) break;
-      }
-      uint32_t avail = end - next;
-      uint32_t r = rank_in_mask(m);
-      bool mine = ((m >> lane_id()) & 1ull) && r < avail;
-      if (mine) id = next + r;
-      uint32_t n = (uint32_t)__popcll(m);
-      uint32_t used = n < avail ? n : avail;
-      next += used;
-      m &= ~__ballot(mine);
-    }
-    return id;
-  }
   // Hands ray ids to the lanes with want == true (all lanes must call).
   // Returns this lane's id, or kNone.
-  __device__ uint32_t take(bool want, uint32_t* queue, uint32_t batch, uint32_t n_rays) {
+  __device__ uint32_t take(bool want, uint32_t* queue, uint32_t batch, uint32_t n_rays, uint32_t unit) {
     uint32_t id = kNone;
     uint64_t m = __ballot(want);
     while (m && !exhausted) {
       if (next >= end) {
-        uint32_t base = 0;
-        if (lane_id() == 0) base = atomicAdd(queue, batch);
-        base = __builtin_amdgcn_readfirstlane(__shfl(base, 0, 64));
-        if (base >= n_rays) {
-          exhausted = true;
-          break;
-        }
-        next = base;
-        end = min(base + batch, n_rays);
+        refill(queue, batch, n_rays, unit);
+        if (exhausted) break;
       }
       uint32_t avail = end - next;
       uint32_t r = rank_in_mask(m);
@@ -790,11 +813,10 @@ __device__ inline bool split_step(Trav& s, Hit& best, Stack<D>& st, Counters& c,
     src = (int)((lane_id() & ~(gsz - 1u)) + nth_set(donors, k % n_d));
   }
   const uint32_t dsp = (uint32_t)__shfl((int)st.sp, src, 64);
-  lds_entry* dl = st.lds;
-  shfl_from(dl, src);
+  const uint32_t dcol = (uint32_t)__shfl((int)st.col, src, 64);
   j3d_u32x2 got = {kNone, 0u};
   const bool take = !busy && depth < dsp;
-  if (take) got = dl[((dsp - 1u - depth) & (D - 1)) * st.stride];
+  if (take) got = st.a.lds[(((dsp - 1u - depth) & (D - 1)) << st.a.shift) + dcol];
   // every receiver has read its entry before any donor refills a slot
   __builtin_amdgcn_wave_barrier();
   if (busy && st.sp > 0u) {
@@ -802,7 +824,7 @@ __device__ inline bool split_step(Trav& s, Hit& best, Stack<D>& st, Counters& c,
     const uint32_t dealt = n_i > r ? (n_i - r + n_d - 1u) / n_d : 0u;
     for (uint32_t i = 0; i < min(dealt, st.sp); ++i) {
       --st.sp;
-      if (st.sp >= (uint32_t)D) st.lds[(st.sp & (D - 1)) * st.stride] = st.spill[(uint64_t)(st.sp - D) * st.sstride];
+      if (st.sp >= (uint32_t)D) *st.slot(st.sp) = *st.spilled(st.sp - D);
     }
   }
   if (take && __uint_as_float(got.y) <= s.thi) s.cur = got.x;
