@@ -254,12 +254,12 @@ __device__ inline void dense(const u32x4* a /* [2 * KB] */, const float* bias, c
 // Output layer: one more row tile whose rows 0 and 1 are W4 (the rest zero);
 // y0, y1 land in registers 0 and 1 of the lane half h = 0 and are broadcast
 // to the other half.
-__device__ inline void output_layer(const Packed* pk, const u32x4* a4, uint32_t lane, const u32x4 h3[4], float& y0,
+__device__ inline void output_layer(const float* b4, const u32x4* a4, uint32_t lane, const u32x4 h3[4], float& y0,
                                     float& y1) {
   const bool h0 = lane < 32;
   f32x16 acc = {};
-  acc[0] = h0 ? pk->b4[0] : 0.f;
-  acc[1] = h0 ? pk->b4[1] : 0.f;
+  acc[0] = h0 ? b4[0] : 0.f;
+  acc[1] = h0 ? b4[1] : 0.f;
 #pragma unroll
   for (int kb = 0; kb < 4; ++kb) acc = mfma(a4[kb], h3[kb], acc);
   y0 = __shfl(acc[0], (int)(lane & 31u), 64);
@@ -294,7 +294,7 @@ __device__ inline void forward(const Packed* pk, const Weights& w, uint32_t lane
   activate(c, h2, m);
   dense<4>(w.a3, pk->bc[2][h], h2, c);
   activate(c, h3, m);
-  output_layer(pk, w.a4, lane, h3, y0, y1);
+  output_layer(pk->b4, w.a4, lane, h3, y0, y1);
 }
 
 // -------------------------------------------------------------- inference ---
@@ -429,6 +429,13 @@ struct ChunkTiles {
   uint16_t in3[64 * kRS];   // h3 (output layer, VALU)
   float dy[2][32];
 };
+// The packed network's biases and output layer, in the order Packed holds them.
+struct Consts {
+  float bc[3][2][32];
+  float w4c[2][2][32];
+  float b4[4];
+};
+static_assert(offsetof(Packed, bc) + sizeof(Consts) == sizeof(Packed) && sizeof(Consts) % 4 == 0, "Packed's tail");
 constexpr int kGradTiles = 14;  // gW1: 2 x 3, gW2: 2 x 2, gW3: 2 x 2
 
 __device__ inline uint16_t bf_bits(float x) { return (uint16_t)(pack2(x, 0.f) & 0xFFFFu); }
@@ -461,44 +468,39 @@ __device__ inline float frag_sum(const u32x4& q) {
 }
 
 // dH = W^T bf16(d) (accumulator order in and out); out = mask ? dH : 0.
-__device__ inline void backprop(const u32x4 (*t)[64], uint32_t lane, const float d[32], uint32_t mask, float out[32]) {
+__device__ inline void backprop(const u32x4* t, const float d[32], uint32_t mask, float out[32]) {
   u32x4 dfr[4];
   to_frags(d, dfr);
-  __builtin_amdgcn_sched_barrier(0);
   f32x16 c[2];
 #pragma unroll
   for (int mt = 0; mt < 2; ++mt) {
     f32x16 acc = {};
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) acc = mfma(ldfrag(&t[mt * 4 + kb][lane]), dfr[kb], acc);
+    for (int kb = 0; kb < 4; ++kb) acc = mfma(t[mt * 4 + kb], dfr[kb], acc);
     c[mt] = acc;
   }
 #pragma unroll
   for (int idx = 0; idx < 32; ++idx) out[idx] = ((mask >> idx) & 1u) ? c[idx / 16][idx % 16] : 0.f;
 }
 
-// Forward with per-use weight loads (the accumulators need the registers).
-template <int KB>
-__device__ inline void dense_g(const u32x4 (*a)[64], const float* bias, uint32_t lane, const u32x4* in, f32x16 c[2]) {
-  __builtin_amdgcn_sched_barrier(0);  // keep each layer's weight loads next to their use
-#pragma unroll
-  for (int mt = 0; mt < 2; ++mt) {
-    f32x16 acc = bias_tile(bias, mt);
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb) acc = mfma(ldfrag(&a[mt * KB + kb][lane]), in[kb], acc);
-    c[mt] = acc;
-  }
-}
-
 // One gradient pass over n rays: block b takes `iters` trips of 4 chunks and
 // writes its summed gradient (parameter order) to partial[b] and its loss sum
 // to loss_out[b].  Gradients are of sum(loss) * inv_n.
+//
+// A training batch of 16,384 rays is one trip of 128 blocks, one wave per
+// SIMD: the chain of one trip bounds the launch, not the 1.3 GFLOP.  All 46
+// weight fragments are therefore loaded at the trip's start, under the feature
+// computation (a wave may use all 512 registers here), and the biases and the
+// output layer come from LDS: 24.5 -> 18.5 us against loads next to each use.
 __global__ __launch_bounds__(256, 1) void k_grad(const Packed* __restrict__ pk_arg, float4 norm4,
                                                  const float* __restrict__ rays, const float* __restrict__ labels,
                                                  uint32_t n, uint32_t iters, float inv_n, float* __restrict__ partial,
                                                  float* __restrict__ loss_out) {
   __shared__ ChunkTiles tiles[4];
+  __shared__ Consts cst;
   const uint32_t lane0 = threadIdx.x & 63u, wib0 = threadIdx.x >> 6;
+  for (uint32_t i = threadIdx.x; i < sizeof(Consts) / 4; i += blockDim.x)
+    reinterpret_cast<uint32_t*>(&cst)[i] = reinterpret_cast<const uint32_t*>(pk_arg->bc)[i];
 
   f32x16 acc[4];
   float gbs[4] = {0.f, 0.f, 0.f, 0.f};
@@ -514,6 +516,13 @@ __global__ __launch_bounds__(256, 1) void k_grad(const Packed* __restrict__ pk_a
     asm volatile("" : "+v"(lane), "+v"(wib), "+s"(pk));
     const uint32_t j = lane & 31u, h = lane >> 5;
     ChunkTiles& T = tiles[wib];
+    Weights w;
+    u32x4 t2[8], t3[8];
+    load_weights(pk, lane, w);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t3[i] = ldfrag(&pk->t3[i][lane]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t2[i] = ldfrag(&pk->t2[i][lane]);
     const float nrm[4] = {norm4.x, norm4.y, norm4.z, norm4.w};
     const uint32_t r = ((blockIdx.x * iters + it) * 4u + wib) * 32u + j;
     const bool valid = r < n;
@@ -529,21 +538,16 @@ __global__ __launch_bounds__(256, 1) void k_grad(const Packed* __restrict__ pk_a
     u32x4 fin[5], h1[4], h2[4], h3[4];
     uint32_t m1, m2, m3;
     f32x16 c[2];
+    if (it == 0) __syncthreads();  // the constants are in LDS
     features(x, h, fin);
-    dense_g<5>(pk->f1, pk->bc[0][h], lane, fin, c);
+    dense<5>(w.a1, cst.bc[0][h], fin, c);
     activate(c, h1, m1);
-    dense_g<4>(pk->f2, pk->bc[1][h], lane, h1, c);
+    dense<4>(w.a2, cst.bc[1][h], h1, c);
     activate(c, h2, m2);
-    dense_g<4>(pk->f3, pk->bc[2][h], lane, h2, c);
+    dense<4>(w.a3, cst.bc[2][h], h2, c);
     activate(c, h3, m3);
     float y0, y1;
-    {
-      __builtin_amdgcn_sched_barrier(0);
-      u32x4 a4[4];
-#pragma unroll
-      for (int kb = 0; kb < 4; ++kb) a4[kb] = ldfrag(&pk->f4[kb][lane]);
-      output_layer(pk, a4, lane, h3, y0, y1);
-    }
+    output_layer(cst.b4, w.a4, lane, h3, y0, y1);
     // loss: hit * 10 (y0 - s)^2 + softplus(y1) - hit * y1
     const float e = y0 - s_lab;
     const float dy0 = valid ? 2.f * kRegWeight * hit * e * inv_n : 0.f;
@@ -553,11 +557,11 @@ __global__ __launch_bounds__(256, 1) void k_grad(const Packed* __restrict__ pk_a
     float d3[32], d2[32], d1[32];
 #pragma unroll
     for (int idx = 0; idx < 32; ++idx) {
-      const float dh = pk->w4c[0][h][idx] * dy0 + pk->w4c[1][h][idx] * dy1;
+      const float dh = cst.w4c[0][h][idx] * dy0 + cst.w4c[1][h][idx] * dy1;
       d3[idx] = ((m3 >> idx) & 1u) ? dh : 0.f;
     }
-    backprop(pk->t3, lane, d3, m2, d2);
-    backprop(pk->t2, lane, d2, m1, d1);
+    backprop(t3, d3, m2, d2);
+    backprop(t2, d2, m1, d1);
 
     __syncthreads();  // the previous trip's readers are done with the tiles
     store_t<5>(T.in0, h, j, fin);
@@ -576,10 +580,14 @@ __global__ __launch_bounds__(256, 1) void k_grad(const Packed* __restrict__ pk_a
     // output layer (own chunk, lane = neuron): gW4[o][n] += sum_r dy_o(r) h3[n](r)
     {
       float a0 = 0.f, a1 = 0.f;
-      for (int rr = 0; rr < 32; ++rr) {
-        const float hv = __uint_as_float((uint32_t)T.in3[lane * kRS + rr] << 16);
-        a0 = a0 + T.dy[0][rr] * hv;
-        a1 = a1 + T.dy[1][rr] * hv;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const u32x4 hv = *reinterpret_cast<const u32x4*>(&T.in3[lane * kRS + 8 * q]);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          a0 = a0 + T.dy[0][8 * q + k] * bf_slot(hv, k);
+          a1 = a1 + T.dy[1][8 * q + k] * bf_slot(hv, k);
+        }
       }
       gw4[0] += a0;
       gw4[1] += a1;
@@ -659,32 +667,99 @@ __global__ __launch_bounds__(256, 1) void k_grad(const Packed* __restrict__ pk_a
   }
 }
 
-// Sum of the per-block partial gradients (fixed order), optionally an Adam step.
-__global__ void k_update(const float* __restrict__ partial, uint32_t waves, const float* __restrict__ loss_part,
-                         float* __restrict__ params, float* __restrict__ m, float* __restrict__ v,
-                         float* __restrict__ grad_out, float* __restrict__ loss_out, float loss_scale, float lr,
-                         float c1, float c2, int update) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p < kParams) {
-    float g = 0.f;
-    for (uint32_t w = 0; w < waves; ++w) g += partial[(size_t)w * kParams + p];
-    if (grad_out) grad_out[p] = g;
-    if (update) {
-      // beta1 = 0.9, beta2 = 0.999; 1 - beta as its own literal (1.f - 0.999f is 1.3e-5 off 0.001)
-      const float b1 = 0.9f, b2 = 0.999f, ob1 = 0.1f, ob2 = 0.001f, eps = 1e-8f;
-      const float mm = b1 * m[p] + ob1 * g;
-      const float vv = b2 * v[p] + ob2 * g * g;
-      m[p] = mm;
-      v[p] = vv;
-      params[p] = params[p] - lr * (mm * c1) / (sqrtf(vv * c2) + eps);
+// The places of parameter p in the packed network, as k_pack fills them: the
+// weight fragments as bf16, the biases and the output layer's rows.
+__device__ inline void put_frag(u32x4 (*f)[64], int fragment, int k, int i, uint16_t v) {
+  const int r = k & 15, h = (r >> 2) & 1, slot = (r >> 3) * 4 + (r & 3);  // k = kperm(k / 16, h, slot)
+  reinterpret_cast<uint16_t*>(&f[fragment][32 * h + i])[slot] = v;
+}
+__device__ inline void pack_param(Packed* pk, int p, float w) {
+  const uint16_t v = (uint16_t)(pack2(w, 0.f) & 0xFFFFu);
+  if (p < oB1) {
+    const int row = (p - oW1) / kIn, k = (p - oW1) % kIn;
+    put_frag(pk->f1, (row >> 5) * 5 + (k >> 4), k, row & 31, v);
+  } else if (p >= oW4 && p < oB4) {
+    const int o = (p - oW4) / kH, k = (p - oW4) % kH;
+    put_frag(pk->f4, k >> 4, k, o, v);
+    // accumulator order: k = crow(c / 16, h, c % 16)
+    const int r = k & 31, h = (r >> 2) & 1, c = (k >> 5) * 16 + (r >> 3) * 4 + (r & 3);
+    pk->w4c[o][h][c] = __uint_as_float((uint32_t)v << 16);
+  } else if (p >= oB4) {
+    pk->b4[p - oB4] = w;
+  } else {
+    const int layer = p < oW2 ? 0 : p < oW3 ? 1 : 2;
+    const int woff = layer == 0 ? oW1 : layer == 1 ? oW2 : oW3, boff = layer == 0 ? oB1 : layer == 1 ? oB2 : oB3;
+    if (p >= boff) {
+      const int n = p - boff, r = n & 31, h = (r >> 2) & 1, c = (n >> 5) * 16 + (r >> 3) * 4 + (r & 3);
+      pk->bc[layer][h][c] = w;
+    } else {
+      const int row = (p - woff) / kH, k = (p - woff) % kH;
+      put_frag(layer == 1 ? pk->f2 : pk->f3, (row >> 5) * 4 + (k >> 4), k, row & 31, v);
+      // transposed: rows are the layer's inputs, the reduction runs over its outputs
+      put_frag(layer == 1 ? pk->t2 : pk->t3, (k >> 5) * 4 + (row >> 4), row, k & 31, v);
     }
   }
-  if (p == 0 && loss_out) {
-    float s = 0.f;
-    for (uint32_t w = 0; w < waves; ++w) s += loss_part[w];
-    *loss_out = s * loss_scale;
+}
+
+// Sum of the per-block partial gradients in block order, optionally an Adam
+// step that also writes the changed parameters into the packed network, so
+// that a training step is two launches (k_grad, k_update).
+//
+// The sum's order is fixed (its rounding is the result's), so one thread adds
+// a parameter's partials one after the other; what bounded it was fetching
+// them, one load latency per few rows.  Here a block stages kUpdRows rows of
+// kUpdParams parameters in LDS with all its threads' loads in flight at once,
+// and one wave adds them from there (128 blocks' partials: 33.2 -> 4.9 us, and
+// the 4.8 us launch that packed the network is gone).
+constexpr int kUpdParams = 64, kUpdRows = 128;
+__global__ void __launch_bounds__(256) k_update(const float* __restrict__ partial, uint32_t rows,
+                                                const float* __restrict__ loss_part, float* __restrict__ params,
+                                                float* __restrict__ m, float* __restrict__ v,
+                                                float* __restrict__ grad_out, float* __restrict__ loss_out,
+                                                float loss_scale, float lr, float c1, float c2, int update,
+                                                Packed* __restrict__ packed) {
+  __shared__ float stage[kUpdRows][kUpdParams];
+  __shared__ float lsum[256];
+  const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+  const int p = (int)(blockIdx.x * kUpdParams + lane);
+  const bool sum_loss = blockIdx.x == 0 && loss_out;
+  float g = 0.f, loss = 0.f;
+  for (uint32_t w0 = 0; w0 < rows; w0 += kUpdRows) {
+    const uint32_t n = min(rows - w0, (uint32_t)kUpdRows);
+    float r[kUpdRows / 4];
+#pragma unroll
+    for (int i = 0; i < kUpdRows / 4; ++i) {
+      const uint32_t w = wave + 4u * (uint32_t)i;
+      r[i] = p < kParams && w < n ? partial[(size_t)(w0 + w) * kParams + p] : 0.f;
+    }
+    if (w0) __syncthreads();  // the previous rows have been added
+#pragma unroll
+    for (int i = 0; i < kUpdRows / 4; ++i) stage[wave + 4u * (uint32_t)i][lane] = r[i];
+    if (sum_loss && threadIdx.x < n) lsum[threadIdx.x] = loss_part[w0 + threadIdx.x];
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll 16
+      for (uint32_t w = 0; w < n; ++w) g += stage[w][lane];
+    } else if (wave == 1 && sum_loss && lane == 0) {
+      for (uint32_t w = 0; w < n; ++w) loss += lsum[w];
+    }
+  }
+  if (wave == 1 && sum_loss && lane == 0) *loss_out = loss * loss_scale;
+  if (wave != 0 || p >= kParams) return;
+  if (grad_out) grad_out[p] = g;
+  if (update) {
+    // beta1 = 0.9, beta2 = 0.999; 1 - beta as its own literal (1.f - 0.999f is 1.3e-5 off 0.001)
+    const float b1 = 0.9f, b2 = 0.999f, ob1 = 0.1f, ob2 = 0.001f, eps = 1e-8f;
+    const float mm = b1 * m[p] + ob1 * g;
+    const float vv = b2 * v[p] + ob2 * g * g;
+    m[p] = mm;
+    v[p] = vv;
+    const float np = params[p] - lr * (mm * c1) / (sqrtf(vv * c2) + eps);
+    params[p] = np;
+    if (packed) pack_param(packed, p, np);
   }
 }
+constexpr int kUpdBlocks = (kParams + kUpdParams - 1) / kUpdParams;
 
 // ------------------------------------------------------------ training data ---
 
@@ -836,9 +911,10 @@ int Ctx::launch_mlp_frame(const FrameParams& fp, uint32_t n_obj, const DevObject
 
 namespace {
 
-// Gradient pass (+ optional Adam step) over n rays already on the device;
-// `partial` holds blocks_cap * J3DG_MLP_PARAMS floats, loss_part blocks_cap.
-int grad_pass(Ctx* ctx, const Packed* pk, const float norm[4], const float* rays, const float* labels, uint32_t n,
+// Gradient pass (+ optional Adam step, after which pk holds the new network)
+// over n rays already on the device; `partial` holds blocks_cap *
+// J3DG_MLP_PARAMS floats, loss_part blocks_cap.
+int grad_pass(Ctx* ctx, Packed* pk, const float norm[4], const float* rays, const float* labels, uint32_t n,
               float* partial, float* loss_part, uint32_t blocks_cap, float* params, float* m, float* v, float* grad_out,
               float* loss_out, float lr, float c1, float c2, bool update) {
   const uint32_t chunks = (n + 31u) / 32u;
@@ -848,8 +924,8 @@ int grad_pass(Ctx* ctx, const Packed* pk, const float norm[4], const float* rays
   hipLaunchKernelGGL(k_grad, dim3(blocks), dim3(256), 0, ctx->stream, pk, make_float4(norm[0], norm[1], norm[2], norm[3]),
                      rays, labels, n, iters, 1.f / (float)n, partial, loss_part);
   HIP_TRY(hipGetLastError(), J3DG_ERR_LAUNCH);
-  hipLaunchKernelGGL(k_update, dim3((kParams + 255) / 256), dim3(256), 0, ctx->stream, partial, blocks, loss_part,
-                     params, m, v, grad_out, loss_out, 1.f / (float)n, lr, c1, c2, update ? 1 : 0);
+  hipLaunchKernelGGL(k_update, dim3(kUpdBlocks), dim3(256), 0, ctx->stream, partial, blocks, loss_part, params, m, v,
+                     grad_out, loss_out, 1.f / (float)n, lr, c1, c2, update ? 1 : 0, update ? pk : nullptr);
   HIP_TRY(hipGetLastError(), J3DG_ERR_LAUNCH);
   return J3DG_OK;
 }
@@ -1021,12 +1097,12 @@ int j3dg_train_proposal(j3dg_ctx* hctx, uint32_t slot, const j3dg_train_opts* op
   HIP_CALL(hipMemcpy(params.p, p0.data(), kParams * sizeof(float), hipMemcpyHostToDevice), J3DG_ERR_LAUNCH);
   HIP_CALL(hipMemsetAsync(mom.p, 0, kParams * sizeof(float), ctx->stream), J3DG_ERR_LAUNCH);
   HIP_CALL(hipMemsetAsync(vel.p, 0, kParams * sizeof(float), ctx->stream), J3DG_ERR_LAUNCH);
+  int rc = j3d::pack(ctx, params.as<float>(), packed.p);
+  if (rc) return rc;
   double b1t = 1.0, b2t = 1.0;
   for (uint64_t st = 0; st < steps; ++st) {
     const uint32_t off = (uint32_t)((st % steps_per_epoch) * o.batch);
     const uint32_t nb = std::min<uint32_t>(o.batch, n - off);
-    int rc = j3d::pack(ctx, params.as<float>(), packed.p);
-    if (rc) return rc;
     b1t *= 0.9, b2t *= 0.999;
     const double frac = steps > 1 ? (double)st / (double)(steps - 1) : 1.0;
     const float lr = (float)(o.lr_final + 0.5 * (o.lr - o.lr_final) * (1.0 + std::cos(3.14159265358979 * frac)));
@@ -1036,8 +1112,6 @@ int j3dg_train_proposal(j3dg_ctx* hctx, uint32_t slot, const j3dg_train_opts* op
                         (float)(1.0 / (1.0 - b1t)), (float)(1.0 / (1.0 - b2t)), true);
     if (rc) return rc;
   }
-  int rc = j3d::pack(ctx, params.as<float>(), packed.p);
-  if (rc) return rc;
   HIP_CALL(hipStreamSynchronize(ctx->stream), J3DG_ERR_LAUNCH);
   auto t2 = std::chrono::steady_clock::now();
 
@@ -1224,9 +1298,9 @@ int j3dg_mlp_adam_step(j3dg_ctx* hctx, float* params, float* m, float* v, const 
   HIP_CALL(hipMemcpy(d + 3 * kParams, grads, kParams * sizeof(float), hipMemcpyHostToDevice), J3DG_ERR_LAUNCH);
   const float c1 = (float)(1.0 / (1.0 - std::pow(0.9, (double)step)));
   const float c2 = (float)(1.0 / (1.0 - std::pow(0.999, (double)step)));
-  hipLaunchKernelGGL(k_update, dim3((kParams + 255) / 256), dim3(256), 0, ctx->stream, d + 3 * kParams, 1u,
+  hipLaunchKernelGGL(k_update, dim3(kUpdBlocks), dim3(256), 0, ctx->stream, d + 3 * kParams, 1u,
                      (const float*)nullptr, d, d + kParams, d + 2 * kParams, (float*)nullptr, (float*)nullptr, 1.f, lr,
-                     c1, c2, 1);
+                     c1, c2, 1, (Packed*)nullptr);
   HIP_CALL(hipGetLastError(), J3DG_ERR_LAUNCH);
   HIP_CALL(hipStreamSynchronize(ctx->stream), J3DG_ERR_LAUNCH);
   HIP_CALL(hipMemcpy(params, d, kParams * sizeof(float), hipMemcpyDeviceToHost), J3DG_ERR_LAUNCH);
