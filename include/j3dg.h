@@ -345,7 +345,7 @@ int j3dg_any_hit_rays(j3dg_ctx* ctx, const uint32_t* slots, uint32_t n_slots, co
    rays: n x 8 floats on the context's device; obj, tri, t, u, v: n each on the
    device (none may be NULL); results as j3dg_trace_rays.  At most
    J3DG_MAX_OBJECTS slots.  Its working memory (queue words, counters, object
-   table, traversal-stack spill area) is one fixed 16 MiB array per GPU, held
+   table, traversal-stack spill area) is one fixed 128 MiB array per GPU, held
    until the process ends; a mesh set whose stack bound needs more spill than
    it holds is refused (J3DG_ERR_UNSUPPORTED).  Synchronous.  Calls that
    overlap on one GPU (from several contexts or threads) share that array and

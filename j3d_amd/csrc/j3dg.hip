@@ -1049,7 +1049,11 @@ __global__ void k_clear_proposal(float2* p, uint64_t n) {
 // object table, [8192, end) the traversal-stack spill area.  Host code never
 // names `scratch` itself (in host code the name is a stand-in, not a device
 // address): it uses the address hipGetSymbolAddress returned for the device.
-constexpr size_t kNoAllocScratchBytes = size_t(16) << 20;
+// The spill area bounds the launch's blocks: a 4M-triangle mesh's stack bound
+// asks for ~100 KB per block, so that 16 MiB held 170 blocks, 680 waves for
+// 1,024 SIMDs; 128 MiB hold the full grid of 1,024 (1M incoherent rays: 0.93 ->
+// 0.35 ms).
+constexpr size_t kNoAllocScratchBytes = size_t(128) << 20;
 constexpr size_t kNoAllocCounters = 1024, kNoAllocObjects = 2048, kNoAllocSpill = 8192;
 static_assert(kQueueWords * sizeof(uint32_t) <= kNoAllocCounters, "queue words fit their slot");
 static_assert(kNoAllocObjects + J3DG_MAX_OBJECTS * sizeof(DevObject) <= kNoAllocSpill, "object table fits its slot");
