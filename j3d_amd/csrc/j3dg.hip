@@ -743,6 +743,26 @@ __global__ void __launch_bounds__(256) k_color(FrameParams f, const DevObject* _
   }
 }
 
+// A frame of no objects (j3d/canvas.cpp:744-760, 859-866): every pixel of the
+// rectangle gets the miss fields; mark, r, g, b and the barycentrics keep their
+// values.  One word per thread, so that a wave's store covers 64 consecutive
+// words (five of every eight are written): bound by the 64 MB of lines a 1080p
+// G-buffer holds.  (As rays through k_trace: 163-174 us; so: 21 us.)
+__global__ void __launch_bounds__(256) k_miss(FrameParams f, uint64_t* counters) {
+  const uint32_t n_words = f.x1 >= f.x0 ? (uint32_t)(f.x1 - f.x0 + 1) * 8u : 0u;
+  const uint32_t k = threadIdx.x & 7u;  // word of the pixel; 1, 2: normal, 3: depth, 4: object_id, 7: db_id
+  const uint32_t v = k == 3u ? __float_as_uint(FLT_MAX) : k == 4u ? kMiss : 0u;
+  const bool write = k - 1u < 4u || k == 7u;
+  for (int32_t y = f.y0 + (int32_t)blockIdx.y; y <= f.y1; y += (int32_t)gridDim.y) {
+    uint32_t* row = reinterpret_cast<uint32_t*>(f.gbuf) + 8 * ((size_t)y * f.w + f.x0);
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < n_words; i += gridDim.x * 256)
+      if (write) row[i] = v;
+  }
+  // the frame's primary rays, for the statistics
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0 && f.y1 >= f.y0)
+    counters[0] = (uint64_t)(n_words / 8u) * (uint32_t)(f.y1 - f.y0 + 1);
+}
+
 __global__ void k_reset(uint32_t* queue, uint64_t* counters, uint32_t n_counters) {
   uint32_t i = threadIdx.x;
   for (uint32_t k = i; k < kQueueWords; k += blockDim.x) queue[k] = 0u;
@@ -1442,6 +1462,18 @@ int Ctx::launch_trace(const FrameParams& fp_in, uint32_t max_stack, int width, b
     fp.pixel_cost = tg->pixel_cost;
   }
   HIP_TRY(hipEventRecord(e[0], stream), J3DG_ERR_LAUNCH);
+  if (!fp.n_obj) {
+    if (fp.n_tiles) {
+      const uint32_t words = (uint32_t)(fp.x1 - fp.x0 + 1) * 8u, rows = (uint32_t)(fp.y1 - fp.y0 + 1);
+      hipLaunchKernelGGL(k_miss, dim3((words + 255) / 256, std::min(rows, 65535u)), dim3(256), 0, stream, fp,
+                         d_counters);
+      HIP_TRY(hipGetLastError(), J3DG_ERR_LAUNCH);
+    }
+    HIP_TRY(hipEventRecord(e[1], stream), J3DG_ERR_LAUNCH);
+    HIP_TRY(hipEventRecord(e[6], stream), J3DG_ERR_LAUNCH);
+    HIP_TRY(hipEventRecord(e[7], stream), J3DG_ERR_LAUNCH);
+    return J3DG_OK;
+  }
   const bool color = fp.fused && (fp.flags & (J3DG_TEXTURED | J3DG_VERTEXCOLORS));
   int rc = launch_trace_kernel((color ? kModeFrameColor : kModeFrame) | top, fp, q, rect_px, fp.n_obj, max_stack,
                                width, d_queue);
