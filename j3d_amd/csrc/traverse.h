@@ -767,6 +767,43 @@ __device__ inline void group_best(Hit& best, uint32_t gsz) {
   }
 }
 
+// Idle lanes are dealt round-robin over the donors (masks of the group's
+// lanes): the k-th idle lane takes entry k / n_d from the top of donor k mod
+// n_d, reading it from the donor's LDS column (a stack's top D entries are
+// always there, and no donor gives more than gsz - 1 < D).  Then each donor
+// drops what it gave, moving spilled entries back into the freed slots as pop
+// does.  Called by all lanes of the group; true for a lane that got an entry.
+template <int D>
+__device__ inline bool deal_work(Stack<D>& st, bool busy, uint32_t idle, uint32_t donors, uint32_t gsz,
+                                 j3d_u32x2& got) {
+  const uint32_t j = split_lane(gsz), below = (1u << j) - 1u;
+  const uint32_t n_d = (uint32_t)__popc(donors), n_i = (uint32_t)__popc(idle);
+  int src = (int)lane_id();
+  uint32_t k = 0, depth = 0;
+  if (!busy) {
+    k = (uint32_t)__popc(idle & below);
+    depth = k / n_d;
+    src = (int)((lane_id() & ~(gsz - 1u)) + nth_set(donors, k % n_d));
+  }
+  const uint32_t dsp = (uint32_t)__shfl((int)st.sp, src, 64);
+  const uint32_t dcol = (uint32_t)__shfl((int)st.col, src, 64);
+  got = {kNone, 0u};
+  const bool take = !busy && depth < dsp;
+  if (take) got = st.a.lds[(((dsp - 1u - depth) & (D - 1)) << st.a.shift) + dcol];
+  // every receiver has read its entry before any donor refills a slot
+  __builtin_amdgcn_wave_barrier();
+  if (busy && st.sp > 0u) {
+    const uint32_t r = (uint32_t)__popc(donors & below);
+    const uint32_t dealt = n_i > r ? (n_i - r + n_d - 1u) / n_d : 0u;
+    const uint32_t drop = min(dealt, st.sp);  // fixed before st.sp changes: all that was taken goes
+    for (uint32_t i = 0; i < drop; ++i) {
+      --st.sp;
+      if (st.sp >= (uint32_t)D) *st.slot(st.sp) = *st.spilled(st.sp - D);
+    }
+  }
+  return take;
+}
+
 // One step of every lane of a group in split mode (called by all gsz lanes).
 // Returns true in every lane when the ray's traversal of the object is
 // complete -- every lane idle with an empty stack, or, for an any-hit ray, a
@@ -798,36 +835,8 @@ __device__ inline bool split_step(Trav& s, Hit& best, Stack<D>& st, Counters& c,
     group_best(best, gsz);
     return true;
   }
-  // Idle lanes are dealt round-robin over the donors: the k-th idle lane takes
-  // entry k / n_d from the top of donor k mod n_d, reading it from the
-  // donor's LDS column (a stack's top D entries are always there, and no donor
-  // gives more than gsz - 1 < D).  Then each donor drops what it gave, moving
-  // spilled entries back into the freed slots as pop does.
-  const uint32_t j = split_lane(gsz), below = (1u << j) - 1u;
-  const uint32_t n_d = (uint32_t)__popc(donors), n_i = (uint32_t)__popc(idle);
-  int src = (int)lane_id();
-  uint32_t k = 0, depth = 0;
-  if (!busy) {
-    k = (uint32_t)__popc(idle & below);
-    depth = k / n_d;
-    src = (int)((lane_id() & ~(gsz - 1u)) + nth_set(donors, k % n_d));
-  }
-  const uint32_t dsp = (uint32_t)__shfl((int)st.sp, src, 64);
-  const uint32_t dcol = (uint32_t)__shfl((int)st.col, src, 64);
-  j3d_u32x2 got = {kNone, 0u};
-  const bool take = !busy && depth < dsp;
-  if (take) got = st.a.lds[(((dsp - 1u - depth) & (D - 1)) << st.a.shift) + dcol];
-  // every receiver has read its entry before any donor refills a slot
-  __builtin_amdgcn_wave_barrier();
-  if (busy && st.sp > 0u) {
-    const uint32_t r = (uint32_t)__popc(donors & below);
-    const uint32_t dealt = n_i > r ? (n_i - r + n_d - 1u) / n_d : 0u;
-    for (uint32_t i = 0; i < min(dealt, st.sp); ++i) {
-      --st.sp;
-      if (st.sp >= (uint32_t)D) *st.slot(st.sp) = *st.spilled(st.sp - D);
-    }
-  }
-  if (take && __uint_as_float(got.y) <= s.thi) s.cur = got.x;
+  j3d_u32x2 got;
+  if (deal_work<D>(st, busy, idle, donors, gsz, got) && __uint_as_float(got.y) <= s.thi) s.cur = got.x;
   return false;
 }
 
