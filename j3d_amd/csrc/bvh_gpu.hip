@@ -26,6 +26,7 @@
 #include <cfloat>
 #include <cmath>
 #include <cstring>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -424,10 +425,9 @@ inline float half_area(const float* lo, const float* hi) {
   return a >= 0.f ? a : 0.f;  // NaN boxes cost nothing (they hold no hits)
 }
 
-// Full-sweep SAH over cl[a, b) (b - a >= 2); appends the subtree's internal
-// nodes to `out` (its root first) and returns the root's position there.
-// Children refs: a cluster's own ref, or kPrimBit-free positions in `out`
-// tagged by `tag` (resolved to node indices by the caller).
+// Full-sweep SAH over clusters; a subtree's internal nodes are appended to
+// `out`, its root first.  Children refs: a cluster's own ref, or positions in
+// `out` tagged by kSahTag (resolved to node indices by the caller).
 struct SahNode {
   uint32_t left, right;  // cluster ref, or (kSahTag | position in out)
   uint32_t count;
@@ -435,57 +435,127 @@ struct SahNode {
 };
 constexpr uint32_t kSahTag = 0x40000000u;
 
-inline uint32_t sah_build(std::vector<Cluster>& cl, uint32_t a, uint32_t b, std::vector<SahNode>& out,
-                          std::vector<float>& right_area) {
-  const uint32_t pos = (uint32_t)out.size();
-  out.emplace_back();
-  SahNode nd;
+// The clusters are sorted once by centroid on each axis (ties by ref) and the
+// three orders are partitioned down the tree: sorting every node's range on
+// every axis took 50 of the 61 ms that loading a 2M-triangle mesh took.  Ranges
+// [a, b) of all arrays belong to one node, so that subtrees can be built by
+// several threads at once.
+struct SahSpace {
+  std::vector<uint32_t> order[3];  // cluster numbers
+  std::vector<uint32_t> tmp;
+  std::vector<float> right_area;   // of clusters [i, b) in an order
+  std::vector<uint8_t> left;       // per cluster: side of the node's split
+  explicit SahSpace(uint32_t m) : tmp(m), right_area(m + 1), left(m) {
+    for (auto& o : order) o.resize(m);
+  }
+};
+
+inline void sah_sort(const std::vector<Cluster>& cl, SahSpace& sp, int axis, uint32_t a, uint32_t b) {
+  // keys in order of (centroid, ref), so that a comparison reads one place: the
+  // centroid's bits made to compare as integers (not a number sorts last)
+  std::vector<std::pair<uint64_t, uint32_t>> keys(b - a);
+  for (uint32_t i = a; i < b; ++i) {
+    float c = cl[i].c[axis];
+    if (!(c == c)) c = INFINITY;
+    c += 0.f;  // -0 becomes 0
+    uint32_t bits;
+    memcpy(&bits, &c, 4);
+    bits = (bits & 0x80000000u) ? ~bits : (bits | 0x80000000u);
+    keys[i - a] = {(uint64_t)bits << 32 | cl[i].ref, i};
+  }
+  std::sort(keys.begin(), keys.end());
+  for (uint32_t i = a; i < b; ++i) sp.order[axis][i] = keys[i - a].second;
+}
+
+// lo, hi: the box so far, never NaN; a NaN bound of c does not count (as fminf
+// and fmaxf, whose calls were most of the sweeps' time).
+inline void grow(float* lo, float* hi, const Cluster& c) {
+  for (int k = 0; k < 3; ++k) lo[k] = c.lo[k] < lo[k] ? c.lo[k] : lo[k], hi[k] = c.hi[k] > hi[k] ? c.hi[k] : hi[k];
+}
+
+// The best split of the node over [a, b) on one axis: the least cost of the
+// positions before a + 1 .. b - 1, ties going to the position nearest the middle
+// (equal boxes: a balanced tree), started from `cost` and `mid`.  True when better.
+inline bool sah_sweep(const std::vector<Cluster>& cl, const std::vector<uint32_t>& o, std::vector<float>& right_area,
+                      uint32_t a, uint32_t b, double& best_cost, uint32_t& best_mid) {
+  float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+  double cnt = 0.0;
+  for (uint32_t i = b; i-- > a + 1;) {  // right_area[i]: clusters [i, b)
+    const Cluster& c = cl[o[i]];
+    grow(lo, hi, c);
+    cnt += c.count;
+    right_area[i] = (float)((double)half_area(lo, hi) * cnt);
+  }
+  for (int k = 0; k < 3; ++k) lo[k] = INFINITY, hi[k] = -INFINITY;
+  cnt = 0.0;
+  const uint32_t centre = a + (b - a) / 2;
+  bool better = false;
+  for (uint32_t i = a; i + 1 < b; ++i) {  // split before i + 1
+    const Cluster& c = cl[o[i]];
+    grow(lo, hi, c);
+    cnt += c.count;
+    const double cost = (double)half_area(lo, hi) * cnt + (double)right_area[i + 1];
+    const uint32_t dm = i + 1 > centre ? i + 1 - centre : centre - (i + 1);
+    const uint32_t db = best_mid > centre ? best_mid - centre : centre - best_mid;
+    if (cost < best_cost || (cost == best_cost && dm < db)) best_cost = cost, best_mid = i + 1, better = true;
+  }
+  return better;
+}
+
+// Splits the node over [a, b): fills its count and box, leaves its halves in
+// [a, mid) and [mid, b) of all three orders and returns mid.
+inline uint32_t sah_split(const std::vector<Cluster>& cl, SahSpace& sp, uint32_t a, uint32_t b, SahNode& nd) {
   nd.count = 0;
   for (int k = 0; k < 3; ++k) nd.lo[k] = INFINITY, nd.hi[k] = -INFINITY;
   for (uint32_t i = a; i < b; ++i) {
-    nd.count += cl[i].count;
-    for (int k = 0; k < 3; ++k) nd.lo[k] = fminf(nd.lo[k], cl[i].lo[k]), nd.hi[k] = fmaxf(nd.hi[k], cl[i].hi[k]);
+    const Cluster& c = cl[sp.order[0][i]];
+    nd.count += c.count;
+    grow(nd.lo, nd.hi, c);
   }
-  // best split over the three centroid orders
-  int best_axis = -1;
-  uint32_t best_mid = a + (b - a) / 2;
-  double best_cost = INFINITY;
-  for (int axis = 0; axis < 3; ++axis) {
-    std::sort(cl.begin() + a, cl.begin() + b, [axis](const Cluster& x, const Cluster& y) {
-      return x.c[axis] < y.c[axis] || (x.c[axis] == y.c[axis] && x.ref < y.ref);
-    });
-    float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    double cnt = 0.0;
-    for (uint32_t i = b; i-- > a + 1;) {  // right_area[i]: clusters [i, b)
-      for (int k = 0; k < 3; ++k) lo[k] = fminf(lo[k], cl[i].lo[k]), hi[k] = fmaxf(hi[k], cl[i].hi[k]);
-      cnt += cl[i].count;
-      right_area[i] = (float)((double)half_area(lo, hi) * cnt);
+  int axis = 0;
+  uint32_t mid = a + (b - a) / 2;
+  double cost = INFINITY;
+  for (int k = 0; k < 3; ++k)
+    if (sah_sweep(cl, sp.order[k], sp.right_area, a, b, cost, mid)) axis = k;
+  const std::vector<uint32_t>& o = sp.order[axis];
+  for (uint32_t i = a; i < b; ++i) sp.left[o[i]] = i < mid ? 1 : 0;
+  for (int k = 0; k < 3; ++k) {
+    if (k == axis) continue;
+    std::vector<uint32_t>& p = sp.order[k];
+    uint32_t l = a, r = mid;
+    for (uint32_t i = a; i < b; ++i) {
+      const uint32_t c = p[i];
+      if (sp.left[c])
+        sp.tmp[l++] = c;
+      else
+        sp.tmp[r++] = c;
     }
-    for (int k = 0; k < 3; ++k) lo[k] = INFINITY, hi[k] = -INFINITY;
-    cnt = 0.0;
-    for (uint32_t i = a; i + 1 < b; ++i) {  // split before i + 1
-      for (int k = 0; k < 3; ++k) lo[k] = fminf(lo[k], cl[i].lo[k]), hi[k] = fmaxf(hi[k], cl[i].hi[k]);
-      cnt += cl[i].count;
-      const double cost = (double)half_area(lo, hi) * cnt + (double)right_area[i + 1];
-      // ties go to the split nearest the middle (equal boxes: a balanced tree)
-      const uint32_t centre = a + (b - a) / 2;
-      const uint32_t dm = i + 1 > centre ? i + 1 - centre : centre - (i + 1);
-      const uint32_t db = best_mid > centre ? best_mid - centre : centre - best_mid;
-      if (cost < best_cost || (cost == best_cost && dm < db)) best_cost = cost, best_axis = axis, best_mid = i + 1;
-    }
+    std::copy(sp.tmp.begin() + a, sp.tmp.begin() + b, p.begin() + a);
   }
-  if (best_axis != 2)  // the last sort was by z
-    std::sort(cl.begin() + a, cl.begin() + b, [best_axis](const Cluster& x, const Cluster& y) {
-      const int ax = best_axis < 0 ? 0 : best_axis;
-      return x.c[ax] < y.c[ax] || (x.c[ax] == y.c[ax] && x.ref < y.ref);
-    });
+  return mid;
+}
+
+// The subtree over [a, b) (b - a >= 2) of sorted orders; returns its root's position in `out`.
+inline uint32_t sah_range(const std::vector<Cluster>& cl, SahSpace& sp, uint32_t a, uint32_t b,
+                          std::vector<SahNode>& out) {
+  const uint32_t pos = (uint32_t)out.size();
+  out.emplace_back();
+  SahNode nd;
+  const uint32_t mid = sah_split(cl, sp, a, b, nd);
   auto side = [&](uint32_t lo_i, uint32_t hi_i) {
-    return hi_i - lo_i == 1 ? cl[lo_i].ref : (kSahTag | sah_build(cl, lo_i, hi_i, out, right_area));
+    return hi_i - lo_i == 1 ? cl[sp.order[0][lo_i]].ref : (kSahTag | sah_range(cl, sp, lo_i, hi_i, out));
   };
-  nd.left = side(a, best_mid);
-  nd.right = side(best_mid, b);
+  nd.left = side(a, mid);
+  nd.right = side(mid, b);
   out[pos] = nd;
   return pos;
+}
+
+inline uint32_t sah_build(std::vector<Cluster>& cl, uint32_t a, uint32_t b, std::vector<SahNode>& out,
+                          std::vector<float>&) {
+  SahSpace sp((uint32_t)cl.size());
+  for (int axis = 0; axis < 3; ++axis) sah_sort(cl, sp, axis, a, b);
+  return sah_range(cl, sp, a, b, out);
 }
 
 __global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
@@ -494,6 +564,54 @@ __global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
 }
 
 }  // namespace lbvh
+
+namespace {
+
+// Runs f on a thread of its own and g on this one; both here when there is no thread to be had.
+template <class F, class G>
+void both(F f, G g) {
+  std::thread th;
+  bool threaded = true;
+  try {
+    th = std::thread(f);
+  } catch (const std::system_error&) {
+    threaded = false;
+  }
+  g();
+  if (threaded)
+    th.join();
+  else
+    f();
+}
+
+// sah_range with subtrees of more than kSahTask clusters built by threads of
+// their own (a 2M-triangle mesh: 16,000-32,000 clusters, a dozen threads).
+constexpr uint32_t kSahTask = 2048;
+uint32_t sah_tasks(const std::vector<lbvh::Cluster>& cl, lbvh::SahSpace& sp, uint32_t a, uint32_t b,
+                   std::vector<lbvh::SahNode>& out) {
+  using namespace lbvh;
+  if (b - a <= kSahTask) return sah_range(cl, sp, a, b, out);
+  const uint32_t pos = (uint32_t)out.size();
+  out.emplace_back();
+  SahNode nd;
+  const uint32_t mid = sah_split(cl, sp, a, b, nd);
+  auto side = [&](uint32_t lo_i, uint32_t hi_i, std::vector<SahNode>& to) {
+    return hi_i - lo_i == 1 ? cl[sp.order[0][lo_i]].ref : (kSahTag | sah_tasks(cl, sp, lo_i, hi_i, to));
+  };
+  std::vector<SahNode> l;
+  uint32_t left = 0;
+  both([&]() { left = side(a, mid, l); }, [&]() { nd.right = side(mid, b, out); });
+  // the left subtree's nodes follow, their positions moved
+  const uint32_t at = (uint32_t)out.size();
+  auto moved = [at](uint32_t r) { return (r & kSahTag) && !(r & kPrimBit) ? r + at : r; };
+  for (SahNode& n : l) n.left = moved(n.left), n.right = moved(n.right);
+  out.insert(out.end(), l.begin(), l.end());
+  nd.left = moved(left);
+  out[pos] = nd;
+  return pos;
+}
+
+}  // namespace
 
 // Device upload and build (j3dg_upload_mesh with J3DG_BUILD_DEVICE).  Fills
 // m's device arrays and info; the vertex and index arrays are copied first.
@@ -528,21 +646,53 @@ int device_build_mesh(Ctx* ctx, Mesh& m, const float* xyz, uint64_t n_vertices, 
     ~Tmp() {
       if (p) hipFree(p);
     }
-  } box, code, code2, index, index2, bnodes, order, q0, q1, counters, sortTmp, last, wide;
+  };
   auto alloc = [&](Tmp& t, size_t bytes) { return hipMalloc(&t.p, std::max<size_t>(bytes, 16)) == hipSuccess; };
+  // One block for the temporaries and one for the mesh's arrays: an allocation
+  // or a release costs ~0.1 ms whatever its size (a 2M-triangle mesh: 23 of
+  // them before; loading and removing it went from 16 to 12 ms).
+  struct Layout {
+    size_t bytes = 0;
+    size_t add(size_t b) {
+      const size_t at = bytes;
+      bytes += (std::max<size_t>(b, 16) + 255) / 256 * 256;
+      return at;
+    }
+  } lt, lm;
   const size_t fb = 3 * (size_t)n * sizeof(float4);
   const size_t tb = 3 * (size_t)n * sizeof(float4);
-  bool ok = hipMalloc(&m.d_verts, std::max<size_t>(3 * n_vertices * sizeof(float), 16)) == hipSuccess &&
-            hipMalloc(&m.d_idx, 3 * (size_t)n * sizeof(uint32_t)) == hipSuccess &&
-            hipMalloc(&m.d_normals, 3 * (size_t)n * sizeof(float)) == hipSuccess &&
-            hipMalloc(&m.d_fin, fb + 3 * sizeof(float4)) == hipSuccess &&
-            hipMalloc(&m.d_tris, tb + 3 * sizeof(float4)) == hipSuccess && alloc(box, 6 * (size_t)n * 4) &&
-            alloc(code, (size_t)n * 8) && alloc(code2, (size_t)n * 8) && alloc(index, (size_t)n * 4) &&
-            alloc(index2, (size_t)n * 4) && alloc(bnodes, (size_t)(n - 1) * sizeof(BNode)) &&
-            alloc(order, (size_t)(n - 1) * 4) &&
-            alloc(q0, (size_t)n * sizeof(Item)) && alloc(q1, (size_t)n * sizeof(Item)) && alloc(counters, 64) &&
-            alloc(last, ((size_t)n + 3) / 4 * 4) && alloc(wide, (size_t)n * words * 4);
-  if (!ok) return ctx->fail(J3DG_ERR_OUT_OF_MEMORY, "device allocation for the device BVH build failed");
+  size_t sort_bytes = 0;
+  {
+    hipcub::DoubleBuffer<uint64_t> k0(nullptr, nullptr);
+    hipcub::DoubleBuffer<uint32_t> v0(nullptr, nullptr);
+    HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, k0, v0, (int)n, 0, 63, st), J3DG_ERR_LAUNCH);
+  }
+  const size_t o_box = lt.add(6 * (size_t)n * 4), o_code = lt.add((size_t)n * 8), o_code2 = lt.add((size_t)n * 8),
+               o_index = lt.add((size_t)n * 4), o_index2 = lt.add((size_t)n * 4),
+               o_bnodes = lt.add((size_t)(n - 1) * sizeof(BNode)), o_order = lt.add((size_t)(n - 1) * 4),
+               o_q0 = lt.add((size_t)n * sizeof(Item)), o_q1 = lt.add((size_t)n * sizeof(Item)),
+               o_counters = lt.add(64), o_last = lt.add(((size_t)n + 3) / 4 * 4),
+               o_wide = lt.add((size_t)n * words * 4), o_sort = lt.add(sort_bytes);
+  const size_t o_verts = lm.add(3 * n_vertices * sizeof(float)), o_idx = lm.add(3 * (size_t)n * sizeof(uint32_t)),
+               o_normals = lm.add(3 * (size_t)n * sizeof(float)), o_fin = lm.add(fb + 3 * sizeof(float4)),
+               o_tris = lm.add(tb + 3 * sizeof(float4));
+  Tmp work;
+  if (hipMalloc(&m.d_block, lm.bytes) != hipSuccess || !alloc(work, lt.bytes))
+    return ctx->fail(J3DG_ERR_OUT_OF_MEMORY, "device allocation for the device BVH build failed");
+  char* const mb = static_cast<char*>(m.d_block);
+  m.d_verts = reinterpret_cast<float*>(mb + o_verts);
+  m.d_idx = reinterpret_cast<uint32_t*>(mb + o_idx);
+  m.d_normals = reinterpret_cast<float*>(mb + o_normals);
+  m.d_fin = reinterpret_cast<float4*>(mb + o_fin);
+  m.d_tris = reinterpret_cast<float4*>(mb + o_tris);
+  struct Part {
+    void* p;
+  };
+  auto part = [&](size_t at) { return Part{static_cast<char*>(work.p) + at}; };
+  const Part box = part(o_box), code = part(o_code), code2 = part(o_code2), index = part(o_index),
+             index2 = part(o_index2), bnodes = part(o_bnodes), order = part(o_order), q0 = part(o_q0),
+             q1 = part(o_q1), counters = part(o_counters), last = part(o_last), wide = part(o_wide),
+             sortTmp = part(o_sort);
   const auto tc = std::chrono::steady_clock::now();
   HIP_TRY(hipMemcpyAsync(m.d_verts, xyz, 3 * n_vertices * sizeof(float), hipMemcpyHostToDevice, st), J3DG_ERR_LAUNCH);
   HIP_TRY(hipMemcpyAsync(m.d_idx, tris, 3 * (size_t)n * sizeof(uint32_t), hipMemcpyHostToDevice, st), J3DG_ERR_LAUNCH);
@@ -565,9 +715,6 @@ int device_build_mesh(Ctx* ctx, Mesh& m, const float* xyz, uint64_t n_vertices, 
   // sort (code, index) pairs
   hipcub::DoubleBuffer<uint64_t> keys((uint64_t*)code.p, (uint64_t*)code2.p);
   hipcub::DoubleBuffer<uint32_t> vals((uint32_t*)index.p, (uint32_t*)index2.p);
-  size_t sort_bytes = 0;
-  HIP_TRY(hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, keys, vals, (int)n, 0, 63, st), J3DG_ERR_LAUNCH);
-  if (!alloc(sortTmp, sort_bytes)) return ctx->fail(J3DG_ERR_OUT_OF_MEMORY, "device sort storage");
   HIP_TRY(hipcub::DeviceRadixSort::SortPairs(sortTmp.p, sort_bytes, keys, vals, (int)n, 0, 63, st), J3DG_ERR_LAUNCH);
   const uint64_t* skeys = keys.Current();
   const uint32_t* sorted = vals.Current();
@@ -625,10 +772,13 @@ int device_build_mesh(Ctx* ctx, Mesh& m, const float* xyz, uint64_t n_vertices, 
     HIP_TRY(hipStreamSynchronize(st), J3DG_ERR_LAUNCH);
     const uint32_t m = mk[0], k = mk[1];
     if (m < 2 || k + 1 != m || m > n) return ctx->fail(J3DG_ERR_INTERNAL, "device BVH build: malformed frontier");
-    Tmp fbox, put_idx, put_val;
-    if (!alloc(fbox, (size_t)m * 8 * sizeof(float)) || !alloc(put_idx, (size_t)k * sizeof(uint32_t)) ||
-        !alloc(put_val, (size_t)k * sizeof(BNode)))
-      return ctx->fail(J3DG_ERR_OUT_OF_MEMORY, "device BVH build: frontier buffers");
+    Layout lf;
+    const size_t o_fbox = lf.add((size_t)m * 8 * sizeof(float)), o_put = lf.add((size_t)k * sizeof(uint32_t)),
+                 o_val = lf.add((size_t)k * sizeof(BNode));
+    Tmp top_work;
+    if (!alloc(top_work, lf.bytes)) return ctx->fail(J3DG_ERR_OUT_OF_MEMORY, "device BVH build: frontier buffers");
+    char* const fw = static_cast<char*>(top_work.p);
+    const Part fbox{fw + o_fbox}, put_idx{fw + o_put}, put_val{fw + o_val};
     hipLaunchKernelGGL(k_frontier_boxes, dim3((m + 255) / 256), dim3(256), 0, st, (const BNode*)bn,
                        (const float*)box.p, sorted, (const uint32_t*)frontier, m, (float*)fbox.p);
     HIP_TRY(hipGetLastError(), J3DG_ERR_LAUNCH);
@@ -647,8 +797,12 @@ int device_build_mesh(Ctx* ctx, Mesh& m, const float* xyz, uint64_t n_vertices, 
     }
     std::vector<SahNode> sn;
     sn.reserve(k);
-    std::vector<float> right_area(m + 1);
-    sah_build(cl, 0, m, sn, right_area);
+    {
+      SahSpace sp(m);
+      both([&]() { both([&]() { sah_sort(cl, sp, 2, 0, m); }, [&]() { sah_sort(cl, sp, 1, 0, m); }); },
+           [&]() { sah_sort(cl, sp, 0, 0, m); });
+      sah_tasks(cl, sp, 0, m, sn);
+    }
     if (sn.size() != k) return ctx->fail(J3DG_ERR_INTERNAL, "device BVH build: top rebuild size");
     // the rebuilt root stays binary node 0; the other rebuilt nodes take the replaced nodes' indices
     std::vector<uint32_t> index_of(k);

@@ -1577,7 +1577,7 @@ static void init_mesh(Mesh& m, uint32_t db_id, const float* cs, const float* xyz
   // for every input (a NaN is skipped by both folds, and the first of equal
   // values is kept), except a NaN in the first vertex, which poisons its axis
   // in the sequential fold and is applied explicitly.
-  const uint64_t per = 1ull << 20;
+  const uint64_t per = 1ull << 16;  // a million vertices on one thread: 3.8 of the 61 ms its mesh took to load
   const uint64_t chunks = (n_vertices + per - 1) / per;
   std::vector<float> part(6 * chunks);
   auto fold = [&](uint64_t c) {

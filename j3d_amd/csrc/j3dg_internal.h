@@ -123,6 +123,7 @@ struct Mesh {
   uint32_t* d_idx = nullptr;
   float* d_normals = nullptr;
   float4* d_fin = nullptr;  // hit completion records (see DevObject::fin)
+  void* d_block = nullptr;  // device-built meshes: one allocation holding the arrays above but d_nodes
   // surface colour (j3d/scene.h:16-18): per-vertex rgb, per-corner uv + texture
   float* d_vcol = nullptr;
   float* d_uv = nullptr;
@@ -136,6 +137,10 @@ struct Mesh {
   bool has_proposal = false;
   void release() {
     if (d_nodes) hipFree(d_nodes);
+    if (d_block) {
+      hipFree(d_block);
+      d_tris = nullptr, d_verts = nullptr, d_idx = nullptr, d_normals = nullptr, d_fin = nullptr, d_block = nullptr;
+    }
     if (d_tris) hipFree(d_tris);
     if (d_verts) hipFree(d_verts);
     if (d_idx) hipFree(d_idx);
