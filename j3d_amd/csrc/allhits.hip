@@ -309,7 +309,9 @@ __global__ void __launch_bounds__(kAllBlock, 4) k_vox_rays(AllHitsArgs a) {
       const uint32_t idle = split_mask(__ballot(!busy), kVoxLanes);
       const uint32_t donors = split_mask(__ballot(busy && st.sp > 0u), kVoxLanes);
       j3d_u32x2 got = {kNone, 0u};
-      if (idle && donors && deal_work<kAllD>(st, busy, idle, donors, kVoxLanes, got)) s.cur = got.x;
+      int src;
+      uint32_t pos;
+      if (idle && donors && deal_work<kAllD>(st, busy, idle, donors, kVoxLanes, got, src, pos)) s.cur = got.x;
     }
     // the group's hits are in memory before its lanes read them
     __threadfence_block();

@@ -42,6 +42,14 @@ enum : uint32_t {
 // 2 -> 0.84, 3 -> 0.80, 4 -> 0.82); with the split tail 4 is (2 -> 0.723-0.728,
 // 3 -> 0.697-0.707, 4 -> 0.679-0.697, 5 -> 0.708-0.712, 6 -> 0.705-0.707).
 constexpr int kStepsPerTrip = 4;
+// Scenes with a top level: a lane done with an object waits for the next walk
+// of the top level, one per kTopWalk steps for all such lanes.  A walk after
+// every step, for whichever lanes need one, ran the walk's code with a few
+// lanes each time (256 objects, 1080p, frames one at a time: 1.43 ms; one walk
+// every 5 steps and the split tail below: 0.94 ms; every 3, 4 and, with one
+// walk per trip, 8 steps: 0.95, 0.94, 1.03 ms).
+constexpr int kTopWalk = 5;
+constexpr int kTopSteps = 10;
 // A cooperative group (the tail with at most 8 rays left in the wave) takes up
 // to kCoopSteps steps per trip: no refill shares its trips any more (28M-
 // triangle frame: 1 -> 0.80 ms, 4 -> 0.78; 8 traversal steps per trip for the
@@ -246,6 +254,7 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
   f4 wo = {0.f, 0.f, 0.f, 1.f}, wd = {0.f, 0.f, 0.f, 0.f};
   Trav s;
   s.any = any_mode;
+  s.at_top = false;
   s.cur = kNone;
   s.obj = 0;
   Hit best;
@@ -260,22 +269,20 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
       s.tmax = best.found ? fminf(best.t, tf) : tf;
       s.thi = s.tmax * kSlackUp;
       s.base = 0;
-      s.cur = 0;  // the top level's root; kNone after this if no object is entered
-      if (top_l)
-        top_next<D>(s, st, lobjs, top_l, f.top_delta, wo, wd);
-      else
-        top_next<D>(s, st, lobjs, top, f.top_delta, wo, wd);
+      s.cur = 0;  // the top level's root
+      s.at_top = true;
+      s.obj = kNone;  // s.r is no object's ray yet (lanes that take work compare the object only)
     } else {
       begin_object(s, lobjs, 0, wo, wd, tn, tf, best);
     }
   };
-  // an object's traversal reported done: unless an any-hit ray has its hit,
-  // the top level supplies the next object
-  auto resume_top = [&](bool done) {
-    if (!kTop || !done || (s.any && best.found)) return done;
-    s.cur = kNone;
-    return top_l ? top_next<D>(s, st, lobjs, top_l, f.top_delta, wo, wd)
-                 : top_next<D>(s, st, lobjs, top, f.top_delta, wo, wd);
+  // walks the lane's part of the top level to the next object; s.cur is kNone if there is none
+  auto walk_top = [&]() {
+    s.at_top = false;
+    if (top_l)
+      top_next<D>(s, st, lobjs, top_l, f.top_delta, wo, wd);
+    else
+      top_next<D>(s, st, lobjs, top, f.top_delta, wo, wd);
   };
   // the tail modes: this lane takes over lane src's ray (all of its state)
   auto take_state = [&](int src) {
@@ -302,6 +309,7 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
     for (uint32_t i = 0; i < k; ++i) free_cols &= free_cols - 1u;
     st.reset((threadIdx.x & ~63u) + (uint32_t)__builtin_ctzll(free_cols));
     s.cur = kNone;
+    s.at_top = false;
   };
 
   for (;;) {
@@ -392,8 +400,8 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
       const uint32_t n_act = (uint32_t)__popcll(act);
       // the split tail (coop_tail 2, 3, 4) starts with 8, 16 or 32 rays left, in
       // groups of 64 / (rays left rounded up to 8, 16, 32) lanes; the
-      // cooperative tail and scenes with a top level wait for 8 rays
-      const uint32_t most = (!kTop && coop_tail >= 2u) ? 8u << (coop_tail - 2u) : 8u;
+      // cooperative tail waits for 8 rays
+      const uint32_t most = coop_tail >= 2u ? 8u << (coop_tail - 2u) : 8u;
       if (n_act > 0 && n_act <= most) {
         // hand each remaining ray to a group of gsz lanes (group g: the g-th active lane)
         gsz = n_act <= 8u ? 8u : n_act <= 16u ? 4u : 2u;
@@ -404,7 +412,7 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
         take_state(has ? (int)__builtin_ctzll(m) : (int)lane_id());
         if (!has) phase = 0u, pix_trips = 0u;
         coop = true;
-        split = !kTop && coop_tail >= 2u;
+        split = coop_tail >= 2u;
         // lanes 1 .. gsz-1 of group g take the free columns (gsz-1)g ..
         // (gsz-1)g + gsz-2 in lane order (the n_act <= 64 / gsz active lanes
         // leave at least (gsz - 1) n_act)
@@ -448,7 +456,10 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
       if (kIsFrame) pix_trips++;
       Counters& cc = (kFrameLike && phase == kShadowPhase) ? cs : c;
       bool done;
-      if (lnobj == 0 || (kTop && phase != kFinishPhase && s.cur == kNone)) {
+      // lanes that start a ray or are done with an object: one walk of the top
+      // level for all of them
+      if (kTop && !split && s.at_top && phase != kFinishPhase) walk_top();
+      if (lnobj == 0 || (kTop && !split && phase != kFinishPhase && s.cur == kNone)) {
         done = true;  // no object, or (top level) no object box on the ray's way or a ray that is not finite
       } else if ((kFrameLike && phase == kFinishPhase) || (W == 8 && !coop)) {
         // one fetch for every lane: a node, a leaf's triangles or a hit's completion record
@@ -474,35 +485,46 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
             s.any = true;
             if (COUNT) ray_steps = 0;
             start_ray(1e-3f, FLT_MAX);
-            if (split && split_lane(gsz) != 0u) s.cur = kNone;  // split mode: lane 0 starts, the others take work
+            if (split && split_lane(gsz) != 0u) s.cur = kNone, s.at_top = false;  // split mode: lane 0 starts, the others take work
           }
         } else {
           if constexpr (W == 8) {
             // up to kStepsPerTrip traversal steps per loop trip: the trip's
             // fixed work (refills, hit completions, bookkeeping: most of its
             // instructions) is shared by more steps
-            done = resume_top(trav_step_fetched<D, COUNT, kTop>(s, best, st, cc, v));
+            done = trav_step_fetched<D, COUNT, kTop>(s, best, st, cc, v);
 #pragma unroll
-            for (int extra = 1; extra < kStepsPerTrip; ++extra) {
-              if (done) break;
+            for (int extra = 1; extra < (kTop ? kTopSteps : kStepsPerTrip); ++extra) {
+              if (kTop && extra % kTopWalk == 0 && done) {
+                if (object_done<D>(s, best, st)) break;
+                walk_top();
+                done = s.cur == kNone;
+              }
+              if (done) {
+                if (kTop) continue;
+                break;
+              }
               const float4* p2 = step_fetch(s);
 #pragma unroll
               for (int k = 0; k < 6; ++k) v[k] = gload4(p2 + k);
-              done = resume_top(trav_step_fetched<D, COUNT, kTop>(s, best, st, cc, v));
+              done = trav_step_fetched<D, COUNT, kTop>(s, best, st, cc, v);
             }
+            if (kTop && done) done = object_done<D>(s, best, st);
           }
         }
       } else if (split) {
         // a group's lanes share `done`: they leave the loop together
-        done = split_step<W, D, COUNT>(s, best, st, cc, gsz);
-        for (int extra = 1; extra < kCoopSteps && !done; ++extra) done = split_step<W, D, COUNT>(s, best, st, cc, gsz);
+        done = false;
+        for (int k = 0; k < kCoopSteps && !done; ++k)
+          done = split_step<W, D, COUNT, kTop>(s, best, st, cc, gsz, lobjs, wo, wd, walk_top);
       } else if (coop) {
         // a group's lanes share `done`: they leave the loop together
-        done = resume_top(coop_step<W, D, COUNT, kTop>(s, best, st, cc));
-        for (int extra = 1; extra < kCoopSteps && !done; ++extra)
-          done = resume_top(coop_step<W, D, COUNT, kTop>(s, best, st, cc));
+        done = coop_step<W, D, COUNT, kTop>(s, best, st, cc);
+        for (int extra = 1; extra < kCoopSteps && !done; ++extra) done = coop_step<W, D, COUNT, kTop>(s, best, st, cc);
+        if (kTop && done) done = object_done<D>(s, best, st);
       } else {
-        done = resume_top(trav_step<W, D, COUNT, kTop>(s, best, st, cc));
+        done = trav_step<W, D, COUNT, kTop>(s, best, st, cc);
+        if (kTop && done) done = object_done<D>(s, best, st);
       }
       if (!kTop && done && !(s.any && best.found) && s.obj + 1 < lnobj) {
         begin_object(s, lobjs, s.obj + 1, wo, wd, s.r.t_near, s.r.t_far, best);
@@ -554,7 +576,7 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
           st.sp = 0;
           const float t0 = frame_ref<M>(f, bp, fi).diagonal / 100.f, tb = s.r.t_far;
           start_ray(tb >= t0 ? tb : t0, FLT_MAX);
-          if (split && split_lane(gsz) != 0u) s.cur = kNone;
+          if (split && split_lane(gsz) != 0u) s.cur = kNone, s.at_top = false;
         } else {
           if (phase == 1) ev |= kEvResolved;
           phase = 0;

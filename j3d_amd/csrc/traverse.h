@@ -331,6 +331,7 @@ struct Trav {
   uint32_t obj; // object index
   uint32_t base;  // scenes with a top level: stack entries below this one are the top level's
   bool any;     // any-hit (shadow) mode
+  bool at_top;  // scenes with a top level: cur is a top-level ref (kNone: pop one)
 };
 
 // A ray whose origin or direction is not finite hits nothing (the triangle
@@ -734,7 +735,8 @@ __device__ inline bool coop_step(Trav& s, Hit& best, Stack<D>& st, Counters& c) 
 // hits stay its own until the group runs out of work; the group's result is
 // then the least hit in the order (t, object, triangle), the order the
 // single-lane traversal keeps, so it does not depend on which lane found what.
-// (Scenes with a top level keep the cooperative tail.)
+// In scenes with a top level a lane may also take a top-level entry, and then
+// walks that part of the top level and its objects.
 
 __device__ inline uint32_t split_lane(uint32_t gsz) { return lane_id() & (gsz - 1u); }
 // bits of the lanes of this lane's group in a wave-wide mask
@@ -773,12 +775,13 @@ __device__ inline void group_best(Hit& best, uint32_t gsz) {
 // always there, and no donor gives more than gsz - 1 < D).  Then each donor
 // drops what it gave, moving spilled entries back into the freed slots as pop
 // does.  Called by all lanes of the group; true for a lane that got an entry.
+// `src` is the lane it came from and `pos` its place in that lane's stack.
 template <int D>
 __device__ inline bool deal_work(Stack<D>& st, bool busy, uint32_t idle, uint32_t donors, uint32_t gsz,
-                                 j3d_u32x2& got) {
+                                 j3d_u32x2& got, int& src, uint32_t& pos) {
   const uint32_t j = split_lane(gsz), below = (1u << j) - 1u;
   const uint32_t n_d = (uint32_t)__popc(donors), n_i = (uint32_t)__popc(idle);
-  int src = (int)lane_id();
+  src = (int)lane_id();
   uint32_t k = 0, depth = 0;
   if (!busy) {
     k = (uint32_t)__popc(idle & below);
@@ -789,7 +792,8 @@ __device__ inline bool deal_work(Stack<D>& st, bool busy, uint32_t idle, uint32_
   const uint32_t dcol = (uint32_t)__shfl((int)st.col, src, 64);
   got = {kNone, 0u};
   const bool take = !busy && depth < dsp;
-  if (take) got = st.a.lds[(((dsp - 1u - depth) & (D - 1)) << st.a.shift) + dcol];
+  pos = dsp - 1u - depth;
+  if (take) got = st.a.lds[((pos & (D - 1)) << st.a.shift) + dcol];
   // every receiver has read its entry before any donor refills a slot
   __builtin_amdgcn_wave_barrier();
   if (busy && st.sp > 0u) {
@@ -802,42 +806,6 @@ __device__ inline bool deal_work(Stack<D>& st, bool busy, uint32_t idle, uint32_
     }
   }
   return take;
-}
-
-// One step of every lane of a group in split mode (called by all gsz lanes).
-// Returns true in every lane when the ray's traversal of the object is
-// complete -- every lane idle with an empty stack, or, for an any-hit ray, a
-// hit found by any lane -- and best then holds the group's result.
-template <int W, int D, bool COUNT>
-__device__ inline bool split_step(Trav& s, Hit& best, Stack<D>& st, Counters& c, uint32_t gsz) {
-  bool busy = s.cur != kNone;
-  if (busy && trav_step<W, D, COUNT>(s, best, st, c)) {
-    busy = false;  // stack run dry (or an any-hit ray's hit)
-    s.cur = kNone;
-  }
-  if (s.any && split_mask(__ballot(best.found), gsz)) {
-    group_best(best, gsz);
-    return true;
-  }
-  float bt = best.found ? best.t : INFINITY;
-  for (uint32_t m = 1; m < gsz; m <<= 1) bt = fminf(bt, __shfl_xor(bt, (int)m, 64));
-  if (bt < s.tmax) {
-    s.tmax = bt;
-    s.thi = bt * kSlackUp;
-  }
-  const uint32_t idle = split_mask(__ballot(!busy), gsz);
-  const uint32_t donors = split_mask(__ballot(busy && st.sp > 0u), gsz);
-  if (!idle) return false;
-  if (!donors) {
-    // all gsz lanes take part (a group's lanes change phase together); compared
-    // with the lanes present, so that a group could never wait on an absent one
-    if (idle != split_mask(__ballot(true), gsz)) return false;
-    group_best(best, gsz);
-    return true;
-  }
-  j3d_u32x2 got;
-  if (deal_work<D>(st, busy, idle, donors, gsz, got) && __uint_as_float(got.y) <= s.thi) s.cur = got.x;
-  return false;
 }
 
 // ---- scenes of more than J3DG_MAX_OBJECTS objects: a top level ------------
@@ -896,6 +864,15 @@ __device__ inline Ray world_ray(f4 o, f4 d, float tn, float tf) {
   return r;
 }
 
+// Makes object oi the one that s traverses (its ray, nodes and triangles).
+__device__ inline void enter_object(Trav& s, const DevObject* __restrict__ objs, uint32_t oi, f4 wo, f4 wd) {
+  const DevObject& ob = objs[oi];
+  s.r = make_object_ray(ob.inv_cs, wo, wd, s.r.t_near, s.r.t_far);
+  s.nodes = ob.nodes;
+  s.tris = ob.tris;
+  s.obj = oi;
+}
+
 // Walks the top level from s.cur (a top node, or kNone: pop the top level's
 // entries) to the next object whose box the ray enters within the current
 // bound, and starts that object's traversal (s.cur = its root).  Returns true
@@ -936,12 +913,7 @@ __device__ inline bool top_next(Trav& s, Stack<D>& st, const DevObject* __restri
       }
     }
     if (cur & kLeafBit) {
-      const uint32_t oi = cur & kLeafIndexMask;
-      const DevObject& ob = objs[oi];
-      s.r = make_object_ray(ob.inv_cs, wo, wd, w.t_near, w.t_far);
-      s.nodes = ob.nodes;
-      s.tris = ob.tris;
-      s.obj = oi;
+      enter_object(s, objs, cur & kLeafIndexMask, wo, wd);
       s.base = st.sp;
       s.cur = 0;  // the object's root, an internal node
       return false;
@@ -959,6 +931,70 @@ __device__ inline bool top_next(Trav& s, Stack<D>& st, const DevObject* __restri
     if (e1 != INFINITY) st.push(r1, e1);
     cur = e0 != INFINITY ? r0 : kNone;
   }
+}
+
+// A traversal of an object reported done: with top-level entries left on the
+// stack (or rather below it), the lane goes on with the top level.
+template <int D>
+__device__ inline bool object_done(Trav& s, const Hit& best, const Stack<D>& st) {
+  s.cur = kNone;
+  if ((s.any && best.found) || st.sp == 0u) return true;
+  s.at_top = true;
+  return false;
+}
+
+// One step of every lane of a group in split mode (called by all gsz lanes).
+// Returns true in every lane when the ray's traversal of the object (of all
+// objects, with a top level) is complete -- every lane idle with an empty
+// stack, or, for an any-hit ray, a hit found by any lane -- and best then
+// holds the group's result.  walk_top: top_next on the lane's state.
+template <int W, int D, bool COUNT, bool TOP, class F>
+__device__ inline bool split_step(Trav& s, Hit& best, Stack<D>& st, Counters& c, uint32_t gsz,
+                                  const DevObject* __restrict__ objs, f4 wo, f4 wd, F walk_top) {
+  if (TOP && s.at_top) walk_top();
+  bool busy = s.cur != kNone;
+  if (busy && trav_step<W, D, COUNT, TOP>(s, best, st, c)) {
+    // stack run dry (or an any-hit ray's hit)
+    busy = TOP && !object_done<D>(s, best, st);
+    s.cur = kNone;  // at_top: every entry left is the top level's (base = sp)
+  }
+  if (s.any && split_mask(__ballot(best.found), gsz)) {
+    group_best(best, gsz);
+    return true;
+  }
+  float bt = best.found ? best.t : INFINITY;
+  for (uint32_t m = 1; m < gsz; m <<= 1) bt = fminf(bt, __shfl_xor(bt, (int)m, 64));
+  if (bt < s.tmax) {
+    s.tmax = bt;
+    s.thi = bt * kSlackUp;
+  }
+  const uint32_t idle = split_mask(__ballot(!busy), gsz);
+  const uint32_t donors = split_mask(__ballot(busy && st.sp > 0u), gsz);
+  if (!idle) return false;
+  if (!donors) {
+    // all gsz lanes take part (a group's lanes change phase together); compared
+    // with the lanes present, so that a group could never wait on an absent one
+    if (idle != split_mask(__ballot(true), gsz)) return false;
+    group_best(best, gsz);
+    return true;
+  }
+  j3d_u32x2 got;
+  int src;
+  uint32_t pos;
+  const bool take = deal_work<D>(st, busy, idle, donors, gsz, got, src, pos);
+  if constexpr (TOP) {
+    const uint32_t base = (uint32_t)__shfl((int)s.base, src, 64), obj = (uint32_t)__shfl((int)s.obj, src, 64);
+    if (busy) s.base = min(s.base, st.sp);  // entries below it may have been given away
+    if (take && __uint_as_float(got.y) <= s.thi) {
+      s.cur = got.x;
+      s.base = 0;
+      s.at_top = pos < base;
+      if (!s.at_top && obj != s.obj) enter_object(s, objs, obj, wo, wd);
+    }
+  } else if (take && __uint_as_float(got.y) <= s.thi) {
+    s.cur = got.x;
+  }
+  return false;
 }
 
 }  // namespace j3d
