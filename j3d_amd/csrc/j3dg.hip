@@ -785,6 +785,8 @@ __global__ void __launch_bounds__(256) k_miss(FrameParams f, uint64_t* counters)
     counters[0] = (uint64_t)(n_words / 8u) * (uint32_t)(f.y1 - f.y0 + 1);
 }
 
+constexpr uint32_t kCounters = 32;
+
 __global__ void k_reset(uint32_t* queue, uint64_t* counters, uint32_t n_counters) {
   uint32_t i = threadIdx.x;
   for (uint32_t k = i; k < kQueueWords; k += blockDim.x) queue[k] = 0u;
@@ -863,7 +865,17 @@ __device__ inline void shade_pixel(const ShadeParams& s, uint32_t x, uint32_t y)
   s.rgba[(size_t)y * s.w + x] = out;
 }
 
-__global__ void __launch_bounds__(256) k_shade(ShadeParams s) {
+// The first block also leaves the queue and the counters as k_reset does, the
+// frame's counters moved to the words behind them, so that the next frame
+// needs no launch for it (1024x768: 202 -> 199 us, frames on three streams).
+__global__ void __launch_bounds__(256) k_shade(ShadeParams s, uint32_t* queue, uint64_t* counters) {
+  if (blockIdx.x == 0 && blockIdx.y == 0) {
+    for (uint32_t k = threadIdx.x; k < kQueueWords; k += blockDim.x) queue[k] = 0u;
+    if (threadIdx.x < kCounters) {
+      counters[kCounters + threadIdx.x] = counters[threadIdx.x];
+      counters[threadIdx.x] = 0ull;
+    }
+  }
   const uint32_t x = blockIdx.x * 64 + (threadIdx.x & 63);
   const uint32_t y = blockIdx.y * 4 + (threadIdx.x >> 6);
   if (x >= s.w || y >= s.h) return;
@@ -1492,8 +1504,6 @@ int Ctx::launch_trace(const FrameParams& fp_in, uint32_t max_stack, int width, b
       HIP_TRY(hipGetLastError(), J3DG_ERR_LAUNCH);
     }
     HIP_TRY(hipEventRecord(e[1], stream), J3DG_ERR_LAUNCH);
-    HIP_TRY(hipEventRecord(e[6], stream), J3DG_ERR_LAUNCH);
-    HIP_TRY(hipEventRecord(e[7], stream), J3DG_ERR_LAUNCH);
     return J3DG_OK;
   }
   const bool color = fp.fused && (fp.flags & (J3DG_TEXTURED | J3DG_VERTEXCOLORS));
@@ -1525,8 +1535,7 @@ int Ctx::launch_trace(const FrameParams& fp_in, uint32_t max_stack, int width, b
     tg->order_rect[0] = fp.x0, tg->order_rect[1] = fp.y0, tg->order_rect[2] = fp.x1, tg->order_rect[3] = fp.y1;
   }
   HIP_TRY(hipEventRecord(e[1], stream), J3DG_ERR_LAUNCH);
-  HIP_TRY(hipEventRecord(e[6], stream), J3DG_ERR_LAUNCH);
-  if (fp.n_obj && !fp.fused) {
+  if (!fp.fused) {
     const bool shadow = (fp.flags & J3DG_SHADOW) != 0;
     if (shadow) {
       rc = ensure_shadow_queue(rect_px);
@@ -1548,14 +1557,20 @@ int Ctx::launch_trace(const FrameParams& fp_in, uint32_t max_stack, int width, b
       if (rc) return rc;
     }
   }
-  HIP_TRY(hipEventRecord(e[7], stream), J3DG_ERR_LAUNCH);
+  if (!fp.fused) {
+    HIP_TRY(hipEventRecord(e[5], stream), J3DG_ERR_LAUNCH);
+    split_pass = true;
+  }
   return J3DG_OK;
 }
 
 int Ctx::reset_counters() {
   Ctx* ctx = this;
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, stream, d_queue, d_counters, 32u);
-  HIP_TRY(hipGetLastError(), J3DG_ERR_LAUNCH);
+  if (!reset_done) {
+    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, stream, d_queue, d_counters, kCounters);
+    HIP_TRY(hipGetLastError(), J3DG_ERR_LAUNCH);
+  }
+  reset_done = false;  // the caller's launches use them
   return J3DG_OK;
 }
 
@@ -1563,10 +1578,14 @@ int Ctx::launch_shade(const ShadeParams& sp) {
   Ctx* ctx = this;
   dim3 grid((sp.w + 63) / 64, (sp.h + 3) / 4);
   hipEvent_t* e = cur_ev();
-  HIP_TRY(hipEventRecord(e[2], stream), J3DG_ERR_LAUNCH);
-  hipLaunchKernelGGL(k_shade, grid, dim3(256), 0, stream, sp);
+  // after a trace the pass starts at the trace's last event: an event between
+  // two launches takes ~5 us of the stream (1024x768, one stream: 255 us with six
+  // events, 241 with three)
+  if (!traced) HIP_TRY(hipEventRecord(e[2], stream), J3DG_ERR_LAUNCH);
+  hipLaunchKernelGGL(k_shade, grid, dim3(256), 0, stream, sp, d_queue, d_counters);
   HIP_TRY(hipGetLastError(), J3DG_ERR_LAUNCH);
   HIP_TRY(hipEventRecord(e[3], stream), J3DG_ERR_LAUNCH);
+  reset_done = true;
   return J3DG_OK;
 }
 
@@ -1720,11 +1739,11 @@ int j3dg_create(int device, j3dg_ctx** out) {
     if (hipEventCreate(&e) != hipSuccess) return cleanup(J3DG_ERR_LAUNCH);
   for (auto& e : ctx->splat_ev)
     if (hipEventCreate(&e) != hipSuccess) return cleanup(J3DG_ERR_LAUNCH);
-  ctx->ring.assign(8 * Ctx::kRing, nullptr);
+  ctx->ring.assign(Ctx::kEvents * Ctx::kRing, nullptr);
   for (auto& e : ctx->ring)
     if (hipEventCreate(&e) != hipSuccess) return cleanup(J3DG_ERR_LAUNCH);
   if (hipMalloc(&ctx->d_queue, kQueueWords * sizeof(uint32_t)) != hipSuccess) return cleanup(J3DG_ERR_OUT_OF_MEMORY);
-  if (hipMalloc(&ctx->d_counters, 32 * sizeof(uint64_t)) != hipSuccess) return cleanup(J3DG_ERR_OUT_OF_MEMORY);
+  if (hipMalloc(&ctx->d_counters, 2 * kCounters * sizeof(uint64_t)) != hipSuccess) return cleanup(J3DG_ERR_OUT_OF_MEMORY);
   if (noalloc_scratch_setup(device, &ctx->noalloc_scratch) != J3DG_OK) return cleanup(J3DG_ERR_LAUNCH);
   *out = reinterpret_cast<j3dg_ctx*>(ctx);
   return J3DG_OK;
@@ -1799,13 +1818,24 @@ int j3dg_set_counting(j3dg_ctx* h, int on) {
   return J3DG_OK;
 }
 
+// Stage times of a render (event_flags fl): trace, shade, mlp, finish + shadow pass; 0 for a stage that did not run.
+static void stage_times(const hipEvent_t* e, uint32_t fl, float ms[4]) {
+  const int from[4] = {0, fl & 8u ? 5 : fl & 1u ? 1 : 2, 4, 1}, to[4] = {1, 3, 0, 5};
+  for (int k = 0; k < 4; ++k) {
+    float t = 0.f;
+    ms[k] = (fl >> k & 1u) && hipEventElapsedTime(&t, e[from[k]], e[to[k]]) == hipSuccess ? t : 0.f;
+  }
+}
+
 int j3dg_get_stats(j3dg_ctx* h, j3dg_stats* st) {
   Ctx* ctx = reinterpret_cast<Ctx*>(h);
   CHECK_CTX();
   if (!st) return ctx->fail(J3DG_ERR_INVALID_ARG, "null stats");
   HIP_CALL(hipStreamSynchronize(ctx->stream), J3DG_ERR_LAUNCH);
-  uint64_t c[32];
-  HIP_CALL(hipMemcpy(c, ctx->d_counters, sizeof(c), hipMemcpyDeviceToHost), J3DG_ERR_LAUNCH);
+  uint64_t c[kCounters];
+  // a shaded frame's counters are behind the live ones (k_shade)
+  HIP_CALL(hipMemcpy(c, ctx->d_counters + (ctx->reset_done ? kCounters : 0), sizeof(c), hipMemcpyDeviceToHost),
+           J3DG_ERR_LAUNCH);
   std::memset(st, 0, sizeof(*st));
   st->shadow_node_visits = c[12];
   st->shadow_tri_tests = c[13];
@@ -1828,12 +1858,10 @@ int j3dg_get_stats(j3dg_ctx* h, j3dg_stats* st) {
   st->learned_fallback = c[8];
   st->wave_trips = c[9];
   st->lane_steps = c[10];
-  float ms = 0.f;
   const hipEvent_t* e = ctx->last_ev ? ctx->last_ev : ctx->ev;
-  if (ctx->traced && hipEventElapsedTime(&ms, e[0], e[1]) == hipSuccess) st->trace_ms = ms;
-  if (ctx->shaded && hipEventElapsedTime(&ms, e[2], e[3]) == hipSuccess) st->shade_ms = ms;
-  if (ctx->mlp_ran && hipEventElapsedTime(&ms, e[4], e[5]) == hipSuccess) st->mlp_ms = ms;
-  if (ctx->traced && hipEventElapsedTime(&ms, e[6], e[7]) == hipSuccess) st->shadow_ms = ms;
+  float ms[4];
+  stage_times(e, ctx->event_flags(), ms);
+  st->trace_ms = ms[0], st->shade_ms = ms[1], st->mlp_ms = ms[2], st->shadow_ms = ms[3];
   st->splat_ms = ctx->splat_ms;
   return J3DG_OK;
 }
@@ -1856,13 +1884,13 @@ int j3dg_get_timings(j3dg_ctx* h, float* trace_ms, float* shade_ms, float* mlp_m
   uint32_t first = ctx->ring_n - cnt;
   uint32_t k = 0;
   for (uint32_t i = first; i < ctx->ring_n && k < max; ++i, ++k) {
-    const hipEvent_t* e = &ctx->ring[8 * (i % Ctx::kRing)];
-    uint32_t fl = ctx->ring_flags[i % Ctx::kRing];
-    float ms = 0.f;
-    if (trace_ms) trace_ms[k] = ((fl & 1) && hipEventElapsedTime(&ms, e[0], e[1]) == hipSuccess) ? ms : 0.f;
-    if (shade_ms) shade_ms[k] = ((fl & 2) && hipEventElapsedTime(&ms, e[2], e[3]) == hipSuccess) ? ms : 0.f;
-    if (mlp_ms) mlp_ms[k] = ((fl & 4) && hipEventElapsedTime(&ms, e[4], e[5]) == hipSuccess) ? ms : 0.f;
-    if (shadow_ms) shadow_ms[k] = ((fl & 1) && hipEventElapsedTime(&ms, e[6], e[7]) == hipSuccess) ? ms : 0.f;
+    const hipEvent_t* e = &ctx->ring[Ctx::kEvents * (i % Ctx::kRing)];
+    float ms[4];
+    stage_times(e, ctx->ring_flags[i % Ctx::kRing], ms);
+    if (trace_ms) trace_ms[k] = ms[0];
+    if (shade_ms) shade_ms[k] = ms[1];
+    if (mlp_ms) mlp_ms[k] = ms[2];
+    if (shadow_ms) shadow_ms[k] = ms[3];
   }
   *n = k;
   return J3DG_OK;
@@ -2243,10 +2271,9 @@ int j3dg_render(j3dg_ctx* h, const j3dg_frame_desc* fd, uint32_t target, uint32_
     return ctx->fail(J3DG_ERR_UNSUPPORTED, "learned frames take at most J3DG_MAX_OBJECTS objects");
   if ((stages & J3DG_STAGE_SHADE) && !ctx->d_matcap) return ctx->fail(J3DG_ERR_INVALID_ARG, "no matcap set");
   HIP_CALL(hipSetDevice(ctx->device), J3DG_ERR_NO_DEVICE);
-  ctx->traced = ctx->shaded = ctx->mlp_ran = false;
+  ctx->traced = ctx->shaded = ctx->mlp_ran = ctx->split_pass = false;
   const uint64_t npx = (uint64_t)tg.w * tg.h;
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, ctx->stream, ctx->d_queue, ctx->d_counters, 32u);
-  HIP_CALL(hipGetLastError(), J3DG_ERR_LAUNCH);
+  if (int rc = ctx->reset_counters()) return rc;
   if (stages & J3DG_STAGE_TRACE) {
     if (fd->flags & J3DG_NO_SCENE) {
       hipLaunchKernelGGL(k_no_scene, dim3((unsigned)((npx + 255) / 256)), dim3(256), 0, ctx->stream, tg.gbuf, npx);
@@ -2299,9 +2326,8 @@ int j3dg_render(j3dg_ctx* h, const j3dg_frame_desc* fd, uint32_t target, uint32_
     ctx->shaded = true;
   }
   {
-    uint32_t fl = (ctx->traced ? 1u : 0u) | (ctx->shaded ? 2u : 0u) | (ctx->mlp_ran ? 4u : 0u);
     ctx->last_ev = ctx->cur_ev();
-    ctx->ring_flags[ctx->ring_n % Ctx::kRing] = fl;
+    ctx->ring_flags[ctx->ring_n % Ctx::kRing] = ctx->event_flags();
     ctx->ring_n++;
   }
   if (gbuf_out) HIP_CALL(hipMemcpyAsync(gbuf_out, tg.gbuf, npx * sizeof(j3dg_pixel), hipMemcpyDeviceToHost, ctx->stream), J3DG_ERR_LAUNCH);
@@ -2322,7 +2348,7 @@ static int trace_rays_impl(Ctx* ctx, const uint32_t* slots, uint32_t n_slots, co
     int rc = ctx->build_object_table(slots, n_slots, max_stack, width);
     if (rc) return rc;
   }
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, ctx->stream, ctx->d_queue, ctx->d_counters, 32u);
+  if (int rc = ctx->reset_counters()) return rc;
   float* d_rays = nullptr;
   uint8_t* d_out = nullptr;
   size_t out_bytes = any ? n : n * 20;
@@ -2682,20 +2708,19 @@ int j3dg_render_batch(j3dg_ctx* h, const j3dg_frame_desc* frames, const uint32_t
   // the learned frames' proposals, before the graph (they change with the cameras)
   for (size_t k = 0; k < infer.size(); ++k) {
     const uint32_t i = infer[k];
-    rc = ctx->launch_mlp_frame(fps[i], fps[i].n_obj, ctx->d_bobjs + fps[i].obj_base, k == 0, k + 1 == infer.size());
+    rc = ctx->launch_mlp_frame(fps[i], fps[i].n_obj, ctx->d_bobjs + fps[i].obj_base, k == 0);
     if (rc) return rc;
   }
   hipEvent_t* e = ctx->cur_ev();
   HIP_CALL(hipEventRecord(e[0], ctx->stream), J3DG_ERR_LAUNCH);
+  ctx->reset_done = false;  // the graph resets and uses the queue and the counters
   HIP_CALL(hipGraphLaunch(ctx->graph_exec, ctx->stream), J3DG_ERR_LAUNCH);
   HIP_CALL(hipEventRecord(e[1], ctx->stream), J3DG_ERR_LAUNCH);
-  HIP_CALL(hipEventRecord(e[6], ctx->stream), J3DG_ERR_LAUNCH);
-  HIP_CALL(hipEventRecord(e[7], ctx->stream), J3DG_ERR_LAUNCH);
   ctx->graph_launches++;
-  ctx->traced = true, ctx->shaded = false, ctx->mlp_ran = !infer.empty();
+  ctx->traced = true, ctx->shaded = ctx->split_pass = false, ctx->mlp_ran = !infer.empty();
   ctx->last_ev = e;
   // trace time covers trace + shade; mlp time, every learned frame's network
-  ctx->ring_flags[ctx->ring_n % Ctx::kRing] = infer.empty() ? 1u : 5u;
+  ctx->ring_flags[ctx->ring_n % Ctx::kRing] = ctx->event_flags();
   ctx->ring_n++;
   return J3DG_OK;
 }

@@ -217,16 +217,24 @@ struct Ctx {
   std::string arch;
   std::string last_error;
   hipStream_t stream = nullptr;
-  hipEvent_t ev[8] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
-  // per-render HIP events (primary trace, shade, mlp, finish + shadow trace: start/end),
+  static constexpr int kEvents = 6;
+  hipEvent_t ev[kEvents] = {};
+  // per-render HIP events: 0, 1 trace, 3 end of shading, 4 start of mlp (which ends
+  // at 0), 5 end of the finish + shadow pass (which starts at 1); shading starts at
+  // the last event of the trace, or at 2 if there was none;
   // kept for every render since the last j3dg_reset_timings
   static constexpr uint32_t kRing = 1024;
-  std::vector<hipEvent_t> ring;    // kRing * 8
+  std::vector<hipEvent_t> ring;    // kRing * kEvents
   uint32_t ring_n = 0;             // renders recorded since reset
-  uint32_t ring_flags[kRing];      // bit 0 trace, bit 1 shade, bit 2 mlp
+  uint32_t ring_flags[kRing];      // event_flags of each
   const hipEvent_t* last_ev = nullptr;
-  hipEvent_t* cur_ev() { return ring.empty() ? ev : &ring[8 * (ring_n % kRing)]; }
+  hipEvent_t* cur_ev() { return ring.empty() ? ev : &ring[kEvents * (ring_n % kRing)]; }
   bool traced = false, shaded = false, mlp_ran = false;
+  bool split_pass = false;  // the trace had a finish + shadow pass of its own
+  // bit 0 trace, bit 1 shade, bit 2 mlp, bit 3 finish + shadow pass
+  uint32_t event_flags() const {
+    return (traced ? 1u : 0u) | (shaded ? 2u : 0u) | (mlp_ran ? 4u : 0u) | (split_pass ? 8u : 0u);
+  }
   hipEvent_t splat_ev[2] = {nullptr, nullptr};  // around each k_splat_depth of j3dg_splat_points
   float splat_ms = 0.f;                          // their sum over the last call's clouds
   bool counting = false;
@@ -236,6 +244,8 @@ struct Ctx {
   std::vector<PointCloud> clouds;
   uint32_t* d_queue = nullptr;
   uint64_t* d_counters = nullptr;
+  // k_shade ran last: queue and counters are reset, the frame's counters are the second half of d_counters
+  bool reset_done = false;
   void* noalloc_scratch = nullptr;  // this device's j3dg_trace_rays_device working memory (not owned)
   uint2* spill = nullptr;
   uint64_t spill_entries = 0;
@@ -294,10 +304,9 @@ struct Ctx {
   // learned proposal for the frame's objects into fp.proposal (mlp.hip)
   // the proposal network over a frame's pixels into fp.proposal; objs: the frame's
   // object table (nullptr: the current single-frame table); the render's mlp
-  // events are recorded before the launch when `first`, after it when `last`
-  int launch_mlp_frame(const FrameParams& fp, uint32_t n_obj, const DevObject* objs = nullptr, bool first = true,
-                       bool last = true);
-  int reset_counters();  // work-queue heads and statistics counters
+  // start event is recorded before the launch when `first`
+  int launch_mlp_frame(const FrameParams& fp, uint32_t n_obj, const DevObject* objs = nullptr, bool first = true);
+  int reset_counters();  // work-queue heads and statistics counters, for a launch that follows
   int launch_trace(const FrameParams& fp, uint32_t max_stack, int width, bool learned, Target* tg = nullptr);
   int launch_trace_kernel(int mode, const FrameParams& fp, const RayQuery& q, uint32_t n_rays, uint32_t n_obj,
                           uint32_t max_stack, int width, uint32_t* qcounter, const BatchParams* bp = nullptr);

@@ -895,7 +895,7 @@ void init_params(uint64_t seed, float s0, std::vector<float>& p) {
 
 }  // namespace
 
-int Ctx::launch_mlp_frame(const FrameParams& fp, uint32_t n_obj, const DevObject* objs, bool first, bool last) {
+int Ctx::launch_mlp_frame(const FrameParams& fp, uint32_t n_obj, const DevObject* objs, bool first) {
   Ctx* ctx = this;
   hipEvent_t* e = cur_ev();
   if (first) HIP_TRY(hipEventRecord(e[4], stream), J3DG_ERR_LAUNCH);
@@ -904,7 +904,6 @@ int Ctx::launch_mlp_frame(const FrameParams& fp, uint32_t n_obj, const DevObject
                      (const Packed*)nullptr, make_float4(0.f, 0.f, 0.f, 1.f), (const float*)nullptr, 0u,
                      const_cast<float2*>(fp.proposal));
   HIP_TRY(hipGetLastError(), J3DG_ERR_LAUNCH);
-  if (last) HIP_TRY(hipEventRecord(e[5], stream), J3DG_ERR_LAUNCH);
   mlp_ran = true;
   return J3DG_OK;
 }
