@@ -2708,7 +2708,7 @@ int j3dg_render_batch(j3dg_ctx* h, const j3dg_frame_desc* frames, const uint32_t
   // the learned frames' proposals, before the graph (they change with the cameras)
   for (size_t k = 0; k < infer.size(); ++k) {
     const uint32_t i = infer[k];
-    rc = ctx->launch_mlp_frame(fps[i], fps[i].n_obj, ctx->d_bobjs + fps[i].obj_base, k == 0);
+    rc = ctx->launch_mlp_frame(fps[i], fps[i].n_obj, ctx->d_bobjs + fps[i].obj_base, k == 0, k + 1 == infer.size());
     if (rc) return rc;
   }
   hipEvent_t* e = ctx->cur_ev();

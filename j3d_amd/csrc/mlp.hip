@@ -895,7 +895,7 @@ void init_params(uint64_t seed, float s0, std::vector<float>& p) {
 
 }  // namespace
 
-int Ctx::launch_mlp_frame(const FrameParams& fp, uint32_t n_obj, const DevObject* objs, bool first) {
+int Ctx::launch_mlp_frame(const FrameParams& fp, uint32_t n_obj, const DevObject* objs, bool first, bool) {
   Ctx* ctx = this;
   hipEvent_t* e = cur_ev();
   if (first) HIP_TRY(hipEventRecord(e[4], stream), J3DG_ERR_LAUNCH);
