@@ -188,7 +188,7 @@ typedef struct j3dg_stats {
   float trace_ms;                    /* primary-ray trace kernel (HIP events, last render) */
   float shade_ms;                    /* shading/edge kernel */
   float mlp_ms;                      /* learned proposal inference */
-  float shadow_ms;                   /* k_finish + shadow-ray trace */
+  float shadow_ms;                   /* k_finish + shadow-ray trace (split_passes 1; else 0: part of trace_ms) */
   float splat_ms;                    /* k_splat_depth of the last j3dg_splat_points, summed over its clouds */
 } j3dg_stats;
 

@@ -815,8 +815,8 @@ __device__ inline bool deal_work(Stack<D>& st, bool busy, uint32_t idle, uint32_
 // a child ref with kLeafBit set is an object index.  Its entries share the
 // lane's stack: an object's traversal starts with base = the stack depth, and
 // pops stop there, so when it runs dry the top level's entries are next.  The
-// top level is walked here, inline, when a ray starts and whenever an object
-// is finished; lanes never fetch top-level nodes through the step machinery.
+// top level is walked here (top_next) by the lanes that start a ray or are done
+// with an object, all such lanes of a wave together; lanes never fetch top-level nodes through the step machinery.
 // World boxes are tested widened by `delta` (a bound on how far a hit found
 // in an object's own frame can lie from the world ray, from rounding in the
 // transforms) on top of the usual t slack, so no object with a hit in range
