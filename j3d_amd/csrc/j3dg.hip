@@ -240,6 +240,7 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
   uint32_t n_rays = n_rays_q;
   if (kIsFrame) n_rays = f.n_tiles * 64u;
   if (M == kModeShadow) n_rays = __builtin_amdgcn_readfirstlane(*q.count);
+  const uint32_t unit = band_unit(batch, kIsFrame && f.pixel_cost);
   const bool learned = kIsFrame && (f.flags & J3DG_LEARNED) && f.proposal;
   const bool any_mode = M == kModeAnyRays || M == kModeShadow;
   const bool fused = M == kModeBatch || (kIsFrame && f.fused);
@@ -319,7 +320,7 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
     if (!pool.exhausted && (n_idle >= refill_min || n_idle == 64)) {
       // hand new rays to idle lanes; ids outside the rectangle leave a lane idle, so repeat
       while (__ballot(phase == 0) && !pool.exhausted) {
-        const uint32_t id = pool.take(phase == 0, queue, batch, n_rays, kIsFrame && f.pixel_cost ? kBandBlock : 1u);
+        const uint32_t id = pool.take(phase == 0, queue, batch, n_rays, unit);
         if (id == kNone) continue;
         float tn, tf;
         if (kFrameLike) {

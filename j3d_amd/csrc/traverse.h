@@ -486,15 +486,22 @@ __device__ inline uint32_t rank_in_mask(uint64_t m) {
 // kBandQueue of the queue array: one address takes an atomic every ~13 ns,
 // whoever asks, so a launch of many tiles must not draw them from one counter
 // (a batch of 24 frames, 316,000 tiles: 4.08 ms with one counter, one tile per
-// atomic; 2.44 ms with the bands and share()).  Frames in cost order cut their
-// bands at multiples of kBandBlock tiles (the order is sorted within bands),
-// other launches at any tile.
+// atomic; 2.44 ms with the bands and share()).  Where the bands are cut: band_unit.
 constexpr uint32_t kXcds = 8;
 constexpr uint32_t kBandsPerXcd = 1;  // 2 and 4 (an XCD draining its bands in turn) measured slower
 constexpr uint32_t kBands = kXcds * kBandsPerXcd;
 constexpr uint32_t kBandBlock = 256;
 constexpr uint32_t kBandQueue = 32;
 constexpr uint32_t kQueueWords = kBandQueue + 16 * kBands;
+
+// Tiles at whose multiples a launch's bands are cut: blocks of the order for
+// frames in cost order (they are sorted within bands), work items (`batch` rays)
+// otherwise: cut inside an item, every band ends in a part of one, and a launch
+// of as many items as waves gives some waves two (64x48 frame, items of four
+// tiles: 462 us with bands cut at any tile, 337 at items).
+__host__ __device__ inline uint32_t band_unit(uint32_t batch, bool ordered) {
+  return ordered ? kBandBlock : batch >> 6;
+}
 
 // First ray id (tile position * 64) of band b of n_tiles tiles, bands being
 // cut at multiples of `unit` tiles.
@@ -527,7 +534,7 @@ struct RayPool {
   // frame: 0.74 ms with one, 0.87 ms with two).
   __device__ static uint32_t share(uint32_t left, uint32_t batch, uint32_t unit) {
     const uint32_t waves = (gridDim.x * (blockDim.x >> 6) + kBands - 1u) / kBands;
-    return unit == 1u && left / (16u * batch) >= waves ? 2u : 1u;
+    return unit != kBandBlock && left / (16u * batch) >= waves ? 2u : 1u;
   }
   // Refills [next, end) from the bands (all lanes must call).
   __device__ void refill(uint32_t* queue, uint32_t batch, uint32_t n_rays, uint32_t unit) {
