@@ -24,6 +24,9 @@
 #pragma once
 #include <stdint.h>
 
+#include <exception>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 namespace j3d {

@@ -26,8 +26,7 @@
 #include <cfloat>
 #include <cmath>
 #include <cstring>
-#include <system_error>
-#include <thread>
+#include <new>
 #include <vector>
 
 #include "bvh_build.h"
@@ -478,9 +477,9 @@ constexpr uint32_t kSahTag = 0x40000000u;
 struct SahSpace {
   std::vector<uint32_t> order[3];  // cluster numbers
   std::vector<uint32_t> tmp;
-  std::vector<float> right_area;   // of clusters [i, b) in an order
+  std::vector<float>& right_area;  // of clusters [i, b) in an order
   std::vector<uint8_t> left;       // per cluster: side of the node's split
-  explicit SahSpace(uint32_t m) : tmp(m), right_area(m + 1), left(m) {
+  SahSpace(uint32_t m, std::vector<float>& area) : tmp(m), right_area(area), left(m) {
     for (auto& o : order) o.resize(m);
   }
 };
@@ -586,45 +585,43 @@ inline uint32_t sah_range(const std::vector<Cluster>& cl, SahSpace& sp, uint32_t
   return pos;
 }
 
-inline uint32_t sah_build(std::vector<Cluster>& cl, uint32_t a, uint32_t b, std::vector<SahNode>& out,
-                          std::vector<float>&) {
-  SahSpace sp((uint32_t)cl.size());
-  for (int axis = 0; axis < 3; ++axis) sah_sort(cl, sp, axis, a, b);
-  return sah_range(cl, sp, a, b, out);
-}
-
-__global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
-  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
-    p[i] = v;
-}
-
-}  // namespace lbvh
-
-namespace {
-
-// Runs f on a thread of its own and g on this one; both here when there is no thread to be had.
+// Runs f on a thread of its own and g on this one; both here when there is no
+// thread to be had.  An exception of either (out of memory) reaches the caller
+// once both have ended.
 template <class F, class G>
 void both(F f, G g) {
-  std::thread th;
-  bool threaded = true;
-  try {
-    th = std::thread(f);
-  } catch (const std::system_error&) {
-    threaded = false;
+  struct Joined {
+    std::thread t;
+    ~Joined() {
+      if (t.joinable()) t.join();
+    }
+  };
+  std::exception_ptr failed;
+  {
+    Joined th;
+    bool threaded = true;
+    try {
+      th.t = std::thread([&]() {
+        try {
+          f();
+        } catch (...) {
+          failed = std::current_exception();
+        }
+      });
+    } catch (const std::system_error&) {
+      threaded = false;
+    }
+    g();
+    if (!threaded) f();
   }
-  g();
-  if (threaded)
-    th.join();
-  else
-    f();
+  if (failed) std::rethrow_exception(failed);
 }
 
 // sah_range with subtrees of more than kSahTask clusters built by threads of
 // their own (a 2M-triangle mesh: 16,000-32,000 clusters, a dozen threads).
 constexpr uint32_t kSahTask = 2048;
-uint32_t sah_tasks(const std::vector<lbvh::Cluster>& cl, lbvh::SahSpace& sp, uint32_t a, uint32_t b,
-                   std::vector<lbvh::SahNode>& out) {
-  using namespace lbvh;
+inline uint32_t sah_tasks(const std::vector<Cluster>& cl, SahSpace& sp, uint32_t a, uint32_t b,
+                          std::vector<SahNode>& out) {
   if (b - a <= kSahTask) return sah_range(cl, sp, a, b, out);
   const uint32_t pos = (uint32_t)out.size();
   out.emplace_back();
@@ -646,7 +643,22 @@ uint32_t sah_tasks(const std::vector<lbvh::Cluster>& cl, lbvh::SahSpace& sp, uin
   return pos;
 }
 
-}  // namespace
+// The tree over clusters [a, b) (b - a >= 2; the clusters cl holds), its root first in `out`; right_area: room for
+// cl.size() + 1 values.
+inline uint32_t sah_build(std::vector<Cluster>& cl, uint32_t a, uint32_t b, std::vector<SahNode>& out,
+                          std::vector<float>& right_area) {
+  SahSpace sp((uint32_t)cl.size(), right_area);
+  both([&]() { both([&]() { sah_sort(cl, sp, 2, a, b); }, [&]() { sah_sort(cl, sp, 1, a, b); }); },
+       [&]() { sah_sort(cl, sp, 0, a, b); });
+  return sah_tasks(cl, sp, a, b, out);
+}
+
+__global__ void k_fill_u32(uint32_t* p, uint64_t n, uint32_t v) {
+  for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x)
+    p[i] = v;
+}
+
+}  // namespace lbvh
 
 // Device upload and build (j3dg_upload_mesh with J3DG_BUILD_DEVICE).  Fills
 // m's device arrays and info; the vertex and index arrays are copied first.
@@ -831,12 +843,12 @@ int device_build_mesh(Ctx* ctx, Mesh& m, const float* xyz, uint64_t n_vertices, 
       std::memcpy(&c.ref, f + 7, 4);
     }
     std::vector<SahNode> sn;
-    sn.reserve(k);
-    {
-      SahSpace sp(m);
-      both([&]() { both([&]() { sah_sort(cl, sp, 2, 0, m); }, [&]() { sah_sort(cl, sp, 1, 0, m); }); },
-           [&]() { sah_sort(cl, sp, 0, 0, m); });
-      sah_tasks(cl, sp, 0, m, sn);
+    try {
+      sn.reserve(k);
+      std::vector<float> right_area(m + 1);
+      sah_build(cl, 0, m, sn, right_area);
+    } catch (const std::bad_alloc&) {
+      return ctx->fail(J3DG_ERR_OUT_OF_MEMORY, "device BVH build: host memory for the top levels");
     }
     if (sn.size() != k) return ctx->fail(J3DG_ERR_INTERNAL, "device BVH build: top rebuild size");
     // the rebuilt root stays binary node 0; the other rebuilt nodes take the replaced nodes' indices
