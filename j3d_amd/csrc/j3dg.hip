@@ -199,7 +199,11 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
   constexpr bool kLdsObjects = M != kModeBatch && !kTop;
   __shared__ DevObject s_objs[kLdsObjects ? J3DG_MAX_OBJECTS : 1];
   __shared__ uint32_t s_drained;  // the work bands that this block's waves found drained
-  if (threadIdx.x == 0) s_drained = 0;
+  uint32_t n_rays = n_rays_q;
+  if (kIsFrame) n_rays = f.n_tiles * 64u;
+  if (M == kModeShadow) n_rays = __builtin_amdgcn_readfirstlane(*q.count);
+  const bool ordered = kIsFrame && f.pixel_cost;
+  if (threadIdx.x == 0) s_drained = bands_without_work(n_rays, ordered);
   if (kLdsObjects) {
     n_obj = min(n_obj, (uint32_t)J3DG_MAX_OBJECTS);
     const uint32_t words = n_obj * (uint32_t)(sizeof(DevObject) / 4);
@@ -237,10 +241,7 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
   uint32_t trips_coop = 0;
   RayPool pool;
   pool.init(&s_drained);
-  uint32_t n_rays = n_rays_q;
-  if (kIsFrame) n_rays = f.n_tiles * 64u;
-  if (M == kModeShadow) n_rays = __builtin_amdgcn_readfirstlane(*q.count);
-  const uint32_t unit = band_unit(batch, kIsFrame && f.pixel_cost);
+  const uint32_t unit = band_unit(n_rays, batch, ordered);
   const bool learned = kIsFrame && (f.flags & J3DG_LEARNED) && f.proposal;
   const bool any_mode = M == kModeAnyRays || M == kModeShadow;
   const bool fused = M == kModeBatch || (kIsFrame && f.fused);

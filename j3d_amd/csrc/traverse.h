@@ -494,12 +494,29 @@ constexpr uint32_t kBandBlock = 256;
 constexpr uint32_t kBandQueue = 32;
 constexpr uint32_t kQueueWords = kBandQueue + 16 * kBands;
 
+// A launch of at most this many tiles is one band, the last, and the others are
+// marked as drained from its start: a wave in search of work would else ask eight
+// counters, one after the other, before it knows that there is none left and its
+// split tail may start (W4 any-hit queries: 1 ray 71 us with eight bands, 69 with
+// one, 64 rays 103 and 101; 64x48 frame of one wave per block 173 and 169).  From
+// there on one counter costs the same or more (60,000 rays, 938 tiles: W4 closest
+// 345 and 360).
+constexpr uint32_t kOneBandTiles = 64;
+__host__ __device__ inline bool one_band(uint32_t n_rays, bool ordered) {
+  return !ordered && n_rays <= 64u * kOneBandTiles;
+}
+__host__ __device__ inline uint32_t bands_without_work(uint32_t n_rays, bool ordered) {
+  return one_band(n_rays, ordered) ? (1u << (kBands - 1u)) - 1u : 0u;
+}
+
 // Tiles at whose multiples a launch's bands are cut: blocks of the order for
-// frames in cost order (they are sorted within bands), work items (`batch` rays)
-// otherwise: cut inside an item, every band ends in a part of one, and a launch
-// of as many items as waves gives some waves two (64x48 frame, items of four
-// tiles: 462 us with bands cut at any tile, 337 at items).
-__host__ __device__ inline uint32_t band_unit(uint32_t batch, bool ordered) {
+// frames in cost order (they are sorted within bands), all tiles for a launch of
+// one band, work items (`batch` rays) otherwise: cut inside an item, every band
+// ends in a part of one, and a launch of as many items as waves gives some waves
+// two (64x48 frame, items of four tiles: 462 us with bands cut at any tile, 337 at
+// items).
+__host__ __device__ inline uint32_t band_unit(uint32_t n_rays, uint32_t batch, bool ordered) {
+  if (one_band(n_rays, ordered)) return n_rays ? (n_rays + 63u) >> 6 : 1u;
   return ordered ? kBandBlock : batch >> 6;
 }
 

@@ -2,7 +2,8 @@
 (j3d_amd/csrc/traverse.h), compiled for the CPU from the source: the bands
 cover the rays once and in order, and only a launch's last work item may be a
 part of one -- an item cut by a band's end is one more item, which a launch of
-as many items as waves cannot spare."""
+as many items as waves cannot spare.  A launch of few tiles is one band: all others
+are marked as drained from the start, and no wave asks their counters."""
 import os
 import shutil
 import subprocess
@@ -22,6 +23,8 @@ int main() {
       const uint64_t lo = band_first_ray(b, n_tiles, unit), hi = band_first_ray(b + 1, n_tiles, unit);
       const uint64_t end = hi < n_rays ? hi : n_rays;
       if (lo != at && lo < n_rays) ++bad;
+      if (n_rays <= 64u * 64u && !ordered && (end > lo) == (bands_without_work(n_rays, ordered) >> b & 1u)) ++bad;
+      if (bands_without_work(n_rays, ordered) >> b & 1u && end > lo) ++bad;
       if (end > lo) n_items += (end - lo + batch - 1) / batch, at = end;
     }
     if (at != n_rays || n_items != ((uint64_t)n_rays + batch - 1) / batch) {
@@ -45,7 +48,7 @@ int main() {
 def test_bands_cover_the_rays_in_whole_items(tmp_path):
     s = open(os.path.join(ROOT, "j3d_amd", "csrc", "traverse.h")).read()
     body = s[s.index("constexpr uint32_t kXcds"):s.index("// Wave-local pool of ray ids")]
-    unit = "band_unit(batch, ordered)"
+    unit = "band_unit(n_rays, batch, ordered)"
     src = tmp_path / "bands.cpp"
     src.write_text("#include <cstdint>\n#include <cstdio>\n#include <initializer_list>\n#define __host__\n#define __device__\n" + body
                    + MAIN.replace("UNIT", unit))
