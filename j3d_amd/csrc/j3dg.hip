@@ -502,6 +502,17 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
                 walk_top();
                 done = s.cur == kNone;
               }
+              // Queries go on to the ray's next object at once: a ray misses most of
+              // several objects in one step, and with one object per trip its other
+              // steps would wait (16 objects: 64 rays closest 263 us, so 253, any hit
+              // 160 and 149; 1M rays closest 3.79 ms and 3.44, any hit 1.68 and 1.48;
+              // one object, 1M rays on device buffers: 349.5 and 352.0 us).
+              if ((M == kModeRays || M == kModeAnyRays) && !kTop && done && s.obj + 1 < n_obj &&
+                  !(s.any && best.found)) {
+                begin_object(s, lobjs, s.obj + 1, wo, wd, s.r.t_near, s.r.t_far, best);
+                st.sp = 0;
+                done = false;
+              }
               if (done) {
                 if (kTop) continue;
                 break;
