@@ -917,6 +917,7 @@ __device__ inline bool top_next(Trav& s, Stack<D>& st, const DevObject* __restri
   for (uint32_t guard = 0;; ++guard) {
     if (guard == kTopGuard) {
       st.overflow = true;
+      st.sp = 0;  // a lane without work has an empty stack: what it is dealt later is of an object
       s.cur = kNone;
       return true;
     }

@@ -6,7 +6,7 @@ environment variable names (the CPU emulation in tests/test_emu_scenes.py).
           the LDS stack depth EMU_STACK, bit for bit against the oracle
   steps   an any-hit query of one wave whose rays miss all of 16 objects: the
           loop trips it takes
-  guard   a query over 24 objects with a build whose top-level walks are cut
+  guard   a query over 60 objects with a build whose top-level walks are cut
           off after a few nodes: it has to report the overflow
 
 Exit status 0 when everything holds, 1 otherwise (a memory fault in the
@@ -27,9 +27,9 @@ from j3d_amd import ffi  # noqa: E402
 from scenes import compare_gbuffers, compare_rgba, random_rays  # noqa: E402
 
 
-def scene(r, n, side, seed):
+def scene(r, n, side, seed, parts=None):
     rng = np.random.default_rng(seed)
-    parts = [J.icosphere(2, seed=3, amplitude=0.1), J.torus(24, 12, R=0.8, r=0.3, seed=4)]
+    parts = parts or [J.icosphere(2, seed=3, amplitude=0.1), J.torus(24, 12, R=0.8, r=0.3, seed=4)]
     slots, meshes = [], []
     for i in range(n):
         v, t = parts[i % 2]
@@ -98,10 +98,12 @@ def steps(r):
 
 
 def guard(r):
+    # objects of few nodes and triangles: most top-level entries are no node or record of theirs
+    small = J.icosphere(0, seed=3)
     bad = 0
     for mode in (4, 3, 2, 1, 0):
         r.set_tuning(**dict(r.get_tuning(), coop_tail=mode))
-        slots, meshes = scene(r, 24, 1.2, 9)
+        slots, _ = scene(r, 60, 1.0, 9, [small, small])
         rays = random_rays(1500, 6, np.zeros(3), 2.5)
         for q in (r.trace_rays, r.any_hit):
             try:

@@ -32,3 +32,31 @@ def test_a_query_goes_on_to_the_next_object_within_a_trip(lib):
     """A loop trip has up to four traversal steps; a lane of a query that is
     done with an object uses those left for the next one."""
     _run(lib, "steps")
+
+
+@pytest.mark.parametrize("tail,depth", [("4", "8"), ("3", "16"), ("2", "8"), ("1", "16"), ("0", "8")])
+def test_many_objects_match_the_oracle(lib, tail, depth):
+    """Frames and queries through a top-level tree, and queries over 16 objects."""
+    _run(lib, "tails", EMU_TAIL=tail, EMU_STACK=depth, EMU_CUS="4")
+
+
+def test_a_cut_top_level_walk_reads_nothing_out_of_bounds(tmp_path):
+    """The walk's bound, meant for a malformed tree, brought down to eight nodes
+    in a copy of the source: lanes end in the middle of the top level, and the
+    split tail must not take their entries for an object's."""
+    sources = build_emu.patched_sources
+
+    def cut(out, variant=None):
+        sources(out, variant)
+        p = os.path.join(out, "traverse.h")
+        s = open(p).read()
+        assert s.count("kTopGuard = 1u << 22;") == 1
+        open(p, "w").write(s.replace("kTopGuard = 1u << 22;", "kTopGuard = 8u;"))
+        return out
+
+    build_emu.patched_sources = cut
+    try:
+        lib = build_emu.build(str(tmp_path))
+    finally:
+        build_emu.patched_sources = sources
+    _run(lib, "guard", EMU_CUS="4")
