@@ -193,17 +193,14 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
   constexpr bool kTop = (MODE & kModeTop) != 0;  // more objects than the LDS table: a top-level BVH
   constexpr bool kIsFrame = M == kModeFrame || M == kModeFrameColor;
   constexpr bool kFrameLike = kIsFrame || M == kModeBatch;
+  constexpr bool kQuery = M == kModeRays || M == kModeAnyRays;
   extern __shared__ uint2 lds_stack[];
   // the object table (at most J3DG_MAX_OBJECTS entries outside batches) is read
   // on every ray start and hit completion: keep the block's copy in LDS
   constexpr bool kLdsObjects = M != kModeBatch && !kTop;
   __shared__ DevObject s_objs[kLdsObjects ? J3DG_MAX_OBJECTS : 1];
   __shared__ uint32_t s_drained;  // the work bands that this block's waves found drained
-  uint32_t n_rays = n_rays_q;
-  if (kIsFrame) n_rays = f.n_tiles * 64u;
-  if (M == kModeShadow) n_rays = __builtin_amdgcn_readfirstlane(*q.count);
-  const bool ordered = kIsFrame && f.pixel_cost;
-  if (threadIdx.x == 0) s_drained = bands_without_work(n_rays, ordered);
+  if (threadIdx.x == 0) s_drained = kQuery ? bands_without_work(n_rays_q, kCutQuery) : 0u;
   if (kLdsObjects) {
     n_obj = min(n_obj, (uint32_t)J3DG_MAX_OBJECTS);
     const uint32_t words = n_obj * (uint32_t)(sizeof(DevObject) / 4);
@@ -241,7 +238,9 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
   uint32_t trips_coop = 0;
   RayPool pool;
   pool.init(&s_drained);
-  const uint32_t unit = band_unit(n_rays, batch, ordered);
+  uint32_t n_rays = n_rays_q;
+  if (kIsFrame) n_rays = f.n_tiles * 64u;
+  if (M == kModeShadow) n_rays = __builtin_amdgcn_readfirstlane(*q.count);
   const bool learned = kIsFrame && (f.flags & J3DG_LEARNED) && f.proposal;
   const bool any_mode = M == kModeAnyRays || M == kModeShadow;
   const bool fused = M == kModeBatch || (kIsFrame && f.fused);
@@ -321,7 +320,8 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
     if (!pool.exhausted && (n_idle >= refill_min || n_idle == 64)) {
       // hand new rays to idle lanes; ids outside the rectangle leave a lane idle, so repeat
       while (__ballot(phase == 0) && !pool.exhausted) {
-        const uint32_t id = pool.take(phase == 0, queue, batch, n_rays, unit);
+        const uint32_t id = pool.take(phase == 0, queue, batch, n_rays,
+                                      kQuery ? kCutQuery : kIsFrame && f.pixel_cost ? kCutOrder : kCutItems);
         if (id == kNone) continue;
         float tn, tf;
         if (kFrameLike) {
@@ -507,8 +507,7 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
               // steps would wait (16 objects: 64 rays closest 263 us, so 253, any hit
               // 160 and 149; 1M rays closest 3.79 ms and 3.44, any hit 1.68 and 1.48;
               // one object, 1M rays on device buffers: 349.5 and 352.0 us).
-              if ((M == kModeRays || M == kModeAnyRays) && !kTop && done && s.obj + 1 < n_obj &&
-                  !(s.any && best.found)) {
+              if (kQuery && !kTop && done && s.obj + 1 < n_obj && !(s.any && best.found)) {
                 begin_object(s, lobjs, s.obj + 1, wo, wd, s.r.t_near, s.r.t_far, best);
                 st.sp = 0;
                 done = false;

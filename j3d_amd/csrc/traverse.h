@@ -486,45 +486,45 @@ __device__ inline uint32_t rank_in_mask(uint64_t m) {
 // kBandQueue of the queue array: one address takes an atomic every ~13 ns,
 // whoever asks, so a launch of many tiles must not draw them from one counter
 // (a batch of 24 frames, 316,000 tiles: 4.08 ms with one counter, one tile per
-// atomic; 2.44 ms with the bands and share()).  Where the bands are cut: band_unit.
+// atomic; 2.44 ms with the bands and share()).  Where the bands are cut: band_cut.
 constexpr uint32_t kXcds = 8;
 constexpr uint32_t kBandsPerXcd = 1;  // 2 and 4 (an XCD draining its bands in turn) measured slower
 constexpr uint32_t kBands = kXcds * kBandsPerXcd;
-constexpr uint32_t kBandBlock = 256;
+constexpr uint32_t kBandBlockBits = 8, kBandBlock = 1u << kBandBlockBits;
 constexpr uint32_t kBandQueue = 32;
 constexpr uint32_t kQueueWords = kBandQueue + 16 * kBands;
 
-// A launch of at most this many tiles is one band, the last, and the others are
+// A query of at most this many tiles is one band, the last, and the others are
 // marked as drained from its start: a wave in search of work would else ask eight
 // counters, one after the other, before it knows that there is none left and its
 // split tail may start (W4 any-hit queries: 1 ray 71 us with eight bands, 69 with
-// one, 64 rays 103 and 101; 64x48 frame of one wave per block 173 and 169).  From
-// there on one counter costs the same or more (60,000 rays, 938 tiles: W4 closest
-// 345 and 360).
-constexpr uint32_t kOneBandTiles = 64;
-__host__ __device__ inline bool one_band(uint32_t n_rays, bool ordered) {
-  return !ordered && n_rays <= 64u * kOneBandTiles;
+// one, 64 rays 103 and 101).  From there on one counter costs the same or more
+// (60,000 rays, 938 tiles: W4 closest 345 and 360).  Frames keep their bands (one
+// band: 64x48 178 -> 175 us, 256x192 no difference).
+constexpr uint32_t kOneBandBits = 6, kOneBandTiles = 1u << kOneBandBits;
+enum BandCut : uint32_t { kCutOrder, kCutItems, kCutQuery };  // frames in cost order, other frames and batches, queries
+__host__ __device__ inline bool one_band(uint32_t n_rays, BandCut cut) {
+  return cut == kCutQuery && n_rays <= 64u * kOneBandTiles;
 }
-__host__ __device__ inline uint32_t bands_without_work(uint32_t n_rays, bool ordered) {
-  return one_band(n_rays, ordered) ? (1u << (kBands - 1u)) - 1u : 0u;
+__host__ __device__ inline uint32_t bands_without_work(uint32_t n_rays, BandCut cut) {
+  return one_band(n_rays, cut) ? (1u << (kBands - 1u)) - 1u : 0u;
 }
 
-// Tiles at whose multiples a launch's bands are cut: blocks of the order for
-// frames in cost order (they are sorted within bands), all tiles for a launch of
-// one band, work items (`batch` rays) otherwise: cut inside an item, every band
-// ends in a part of one, and a launch of as many items as waves gives some waves
-// two (64x48 frame, items of four tiles: 462 us with bands cut at any tile, 337 at
-// items).
-__host__ __device__ inline uint32_t band_unit(uint32_t n_rays, uint32_t batch, bool ordered) {
-  if (one_band(n_rays, ordered)) return n_rays ? (n_rays + 63u) >> 6 : 1u;
-  return ordered ? kBandBlock : batch >> 6;
+// Tiles at whose multiples a launch's bands are cut, as a power of two: blocks of
+// the order for frames in cost order (they are sorted within bands), all tiles for
+// a launch of one band, work items (`batch` rays: 1, 2 or 4 tiles) otherwise: cut
+// inside an item, every band ends in a part of one, and a launch of as many items
+// as waves gives some waves two (64x48 frame, items of four tiles: 462 us with bands
+// cut at any tile, 337 at items).
+__host__ __device__ inline uint32_t band_cut(uint32_t n_rays, uint32_t batch, BandCut cut) {
+  return cut == kCutOrder ? kBandBlockBits : one_band(n_rays, cut) ? kOneBandBits : batch >> 7;
 }
 
 // First ray id (tile position * 64) of band b of n_tiles tiles, bands being
-// cut at multiples of `unit` tiles.
+// cut at multiples of 2^unit tiles.
 __host__ __device__ inline uint32_t band_first_ray(uint32_t b, uint32_t n_tiles, uint32_t unit) {
-  const uint32_t nb = (n_tiles + unit - 1) / unit;
-  const uint32_t t = (uint32_t)((uint64_t)b * nb / kBands) * unit;
+  const uint32_t nb = (n_tiles + (1u << unit) - 1u) >> unit;
+  const uint32_t t = (uint32_t)((uint64_t)b * nb / kBands) << unit;
   return (t < n_tiles ? t : n_tiles) * 64u;
 }
 
@@ -549,13 +549,13 @@ struct RayPool {
   // 2.59, 2.86 and 3.58 ms with 4, 8 and 32), and frames in cost order, whose
   // heaviest tiles are neighbours, take one at a time (28M-triangle 1080p
   // frame: 0.74 ms with one, 0.87 ms with two).
-  __device__ static uint32_t share(uint32_t left, uint32_t batch, uint32_t unit) {
+  __device__ static uint32_t share(uint32_t left, uint32_t batch, BandCut cut) {
     const uint32_t waves = (gridDim.x * (blockDim.x >> 6) + kBands - 1u) / kBands;
-    return unit != kBandBlock && left / (16u * batch) >= waves ? 2u : 1u;
+    return cut != kCutOrder && left / (16u * batch) >= waves ? 2u : 1u;
   }
   // Refills [next, end) from the bands (all lanes must call).
-  __device__ void refill(uint32_t* queue, uint32_t batch, uint32_t n_rays, uint32_t unit) {
-    const uint32_t n_tiles = (n_rays + 63u) >> 6;
+  __device__ void refill(uint32_t* queue, uint32_t batch, uint32_t n_rays, BandCut cut) {
+    const uint32_t n_tiles = (n_rays + 63u) >> 6, unit = band_cut(n_rays, batch, cut);
     for (;;) {
       // skip the bands that waves of this block found drained: a failing atomic
       // costs as much as one that brings work, and every wave would make eight
@@ -568,7 +568,7 @@ struct RayPool {
       const uint32_t lo = band_first_ray(band, n_tiles, unit);
       const uint32_t hi = min(band_first_ray(band + 1, n_tiles, unit), n_rays);
       const uint32_t size = hi > lo ? hi - lo : 0u;
-      if (items == 0) items = share(size, batch, unit);
+      if (items == 0) items = share(size, batch, cut);
       const uint32_t amount = items * batch;
       uint32_t base = size;
       if (size) {
@@ -578,7 +578,7 @@ struct RayPool {
       if (base < size) {
         next = lo + base;
         end = hi - next > amount ? next + amount : hi;
-        items = share(size - base, batch, unit);
+        items = share(size - base, batch, cut);
         return;
       }
       if (lane_id() == 0) atomicOr((uint32_t*)drained, 1u << band);
@@ -588,12 +588,12 @@ struct RayPool {
   }
   // Hands ray ids to the lanes with want == true (all lanes must call).
   // Returns this lane's id, or kNone.
-  __device__ uint32_t take(bool want, uint32_t* queue, uint32_t batch, uint32_t n_rays, uint32_t unit) {
+  __device__ uint32_t take(bool want, uint32_t* queue, uint32_t batch, uint32_t n_rays, BandCut cut) {
     uint32_t id = kNone;
     uint64_t m = __ballot(want);
     while (m && !exhausted) {
       if (next >= end) {
-        refill(queue, batch, n_rays, unit);
+        refill(queue, batch, n_rays, cut);
         if (exhausted) break;
       }
       uint32_t avail = end - next;
