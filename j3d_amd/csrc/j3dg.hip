@@ -1614,7 +1614,8 @@ namespace j3d {
 
 // Mesh bookkeeping shared by both builders: pose, bounding box (scene.cpp:22,
 // mesh.cpp:39-58) and a free slot.
-static void init_mesh(Mesh& m, uint32_t db_id, const float* cs, const float* xyz, uint64_t n_vertices, uint64_t n_triangles) {
+static void init_mesh(Mesh& m, uint32_t db_id, const float* cs, const float* xyz, uint64_t n_vertices,
+                      uint64_t n_triangles, int max_threads) {
   m.live = true;
   m.db_id = db_id;
   if (cs)
@@ -1643,17 +1644,21 @@ static void init_mesh(Mesh& m, uint32_t db_id, const float* cs, const float* xyz
       }
     for (int k = 0; k < 3; ++k) part[6 * c + k] = lo[k], part[6 * c + 3 + k] = hi[k];
   };
-  const uint64_t threads = std::min<uint64_t>(chunks, std::max(1u, std::thread::hardware_concurrency()));
-  if (threads <= 1) {
-    for (uint64_t c = 0; c < chunks; ++c) fold(c);
-  } else {
-    std::vector<std::thread> pool;
-    for (uint64_t t = 0; t < threads; ++t)
-      pool.emplace_back([&, t]() {
-        for (uint64_t c = t; c < chunks; c += threads) fold(c);
-      });
-    for (auto& th : pool) th.join();
+  // this thread takes every `threads`-th chunk, and those of threads that were not to be had
+  const uint64_t limit = max_threads > 0 ? max_threads : std::max(1u, std::thread::hardware_concurrency());
+  const uint64_t threads = std::min<uint64_t>(chunks, limit);
+  auto stride = [&](uint64_t t) {
+    for (uint64_t c = t; c < chunks; c += threads) fold(c);
+  };
+  std::vector<std::thread> pool;
+  pool.reserve(threads);
+  try {
+    while (pool.size() + 1 < threads) pool.emplace_back(stride, pool.size() + 1);
+  } catch (const std::exception&) {
   }
+  for (uint64_t t = pool.size() + 1; t < threads; ++t) stride(t);
+  stride(0);
+  for (auto& th : pool) th.join();
   for (int k = 0; k < 3; ++k) {
     float lo = xyz[k], hi = xyz[k];
     for (uint64_t c = 0; c < chunks; ++c) {
@@ -1685,7 +1690,7 @@ static int upload_mesh_device(Ctx* ctx, uint32_t db_id, const float* xyz, uint64
                        uint64_t n_triangles, const float* cs, const BuildOptions& bo, uint32_t* slot) {
   auto t0 = std::chrono::steady_clock::now();
   Mesh m;
-  init_mesh(m, db_id, cs, xyz, n_vertices, n_triangles);
+  init_mesh(m, db_id, cs, xyz, n_vertices, n_triangles, bo.threads);
   double upload_s = 0.0;
   int rc = device_build_mesh(ctx, m, xyz, n_vertices, tris, n_triangles, bo.width, bo.leaf_size, &upload_s);
   if (rc != J3DG_OK) {
@@ -1956,7 +1961,7 @@ int j3dg_upload_mesh(j3dg_ctx* h, uint32_t db_id, const float* xyz, uint64_t n_v
     for (auto& th : pool) th.join();
   }
   Mesh m;
-  j3d::init_mesh(m, db_id, cs, xyz, n_vertices, n_triangles);
+  j3d::init_mesh(m, db_id, cs, xyz, n_vertices, n_triangles, bo.threads);
   m.info.n_nodes = bvh.n_nodes;
   m.info.width = (uint32_t)bvh.width;
   m.info.max_depth = bvh.max_depth;
