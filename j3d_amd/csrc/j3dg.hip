@@ -189,11 +189,12 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
                                                uint32_t spill_cap, uint32_t* queue, uint64_t* counters,
                                                uint32_t batch, uint32_t refill_min, uint32_t coop_tail,
                                                uint64_t* timeline, BatchParams bp) {
-  constexpr int M = MODE & (kModeTop - 1);
+  constexpr int M = MODE & (kModeMany - 1);
   constexpr bool kTop = (MODE & kModeTop) != 0;  // more objects than the LDS table: a top-level BVH
   constexpr bool kIsFrame = M == kModeFrame || M == kModeFrameColor;
   constexpr bool kFrameLike = kIsFrame || M == kModeBatch;
   constexpr bool kQuery = M == kModeRays || M == kModeAnyRays;
+  constexpr bool kMany = (MODE & kModeMany) != 0;  // a query over several objects
   extern __shared__ uint2 lds_stack[];
   // the object table (at most J3DG_MAX_OBJECTS entries outside batches) is read
   // on every ray start and hit completion: keep the block's copy in LDS
@@ -505,9 +506,9 @@ __global__ void __launch_bounds__(256, COUNT ? 1 : 3) k_trace(FrameParams f, Ray
               // Queries go on to the ray's next object at once: a ray misses most of
               // several objects in one step, and with one object per trip its other
               // steps would wait (16 objects: 64 rays closest 263 us, so 253, any hit
-              // 160 and 149; 1M rays closest 3.79 ms and 3.44, any hit 1.68 and 1.48;
-              // one object, 1M rays on device buffers: 349.5 and 352.0 us).
-              if (kQuery && !kTop && done && s.obj + 1 < n_obj && !(s.any && best.found)) {
+              // 160 and 149; 1M rays closest 3.79 ms and 3.44, any hit 1.68 and 1.48).
+              // Kernels of their own: queries of one object lost 1 % to the code.
+              if (kMany && done && s.obj + 1 < n_obj && !(s.any && best.found)) {
                 begin_object(s, lobjs, s.obj + 1, wo, wd, s.r.t_near, s.r.t_far, best);
                 st.sp = 0;
                 done = false;
@@ -1135,16 +1136,16 @@ void* trace_kernel_wd(bool count) {
   return count ? (void*)&k_trace<W, D, true, MODE> : (void*)&k_trace<W, D, false, MODE>;
 }
 
+template <int W, int MODE>
+void* trace_kernel_w(int depth, bool count) {
+  if (depth == 8) return trace_kernel_wd<W, 8, MODE>(count);
+  if (depth == 32) return trace_kernel_wd<W, 32, MODE>(count);
+  return trace_kernel_wd<W, 16, MODE>(count);
+}
+
 template <int MODE>
 void* trace_kernel_mode(int width, int depth, bool count) {
-  if (width == 8) {
-    if (depth == 8) return trace_kernel_wd<8, 8, MODE>(count);
-    if (depth == 32) return trace_kernel_wd<8, 32, MODE>(count);
-    return trace_kernel_wd<8, 16, MODE>(count);
-  }
-  if (depth == 8) return trace_kernel_wd<4, 8, MODE>(count);
-  if (depth == 32) return trace_kernel_wd<4, 32, MODE>(count);
-  return trace_kernel_wd<4, 16, MODE>(count);
+  return width == 8 ? trace_kernel_w<8, MODE>(depth, count) : trace_kernel_w<4, MODE>(depth, count);
 }
 
 void* trace_kernel(int mode, int width, int depth, bool count) {
@@ -1152,6 +1153,8 @@ void* trace_kernel(int mode, int width, int depth, bool count) {
   if (mode == (kModeAnyRays | kModeTop)) return trace_kernel_mode<kModeAnyRays | kModeTop>(width, depth, false);
   if (mode == (kModeFrameColor | kModeTop)) return trace_kernel_mode<kModeFrameColor | kModeTop>(width, depth, count);
   if (mode == (kModeFrame | kModeTop)) return trace_kernel_mode<kModeFrame | kModeTop>(width, depth, count);
+  if (mode == (kModeRays | kModeMany)) return trace_kernel_w<8, kModeRays | kModeMany>(depth, false);
+  if (mode == (kModeAnyRays | kModeMany)) return trace_kernel_w<8, kModeAnyRays | kModeMany>(depth, count);
   if (mode == kModeBatch) return trace_kernel_mode<kModeBatch>(width, depth, count);
   if (mode == kModeRays) return trace_kernel_mode<kModeRays>(width, depth, false);
   if (mode == kModeAnyRays) return trace_kernel_mode<kModeAnyRays>(width, depth, count);
@@ -2407,6 +2410,8 @@ static int trace_rays_impl(Ctx* ctx, const uint32_t* slots, uint32_t n_slots, co
     fp.top_delta = ctx->top_delta(r);
     fp.top_count = ctx->top_count;
     mode |= kModeTop;
+  } else if (n_slots > 1 && width == 8) {
+    mode |= kModeMany;
   }
   int rc = ctx->launch_trace_kernel(mode, fp, q, (uint32_t)n, n_slots, max_stack, width, ctx->d_queue);
   if (rc) return rc;
@@ -2499,7 +2504,7 @@ int j3dg_trace_rays_device(j3dg_ctx* h, const uint32_t* slots, uint32_t n_slots,
   uint32_t batch = 64u * ctx->tuning.rays_per_item, refill = ctx->tuning.refill_min, coop = ctx->tuning.coop_tail;
   uint64_t* tl = nullptr;
   void* args[] = {&f, &q, &nr, &objs_c, &no, &spill, &capv, &queue, &counters, &batch, &refill, &coop, &tl, &bp};
-  void* fn = j3d::trace_kernel(kModeRays, width, (int)D, false);
+  void* fn = j3d::trace_kernel(n_slots > 1 && width == 8 ? kModeRays | kModeMany : kModeRays, width, (int)D, false);
   HIP_CALL(hipLaunchKernel(fn, dim3(grid), dim3(block), args, D * block * sizeof(uint2), ctx->stream),
            J3DG_ERR_LAUNCH);
   uint64_t overflow = 0;

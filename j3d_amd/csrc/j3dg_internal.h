@@ -68,6 +68,8 @@ enum { kModeFrame = 0, kModeRays = 1, kModeAnyRays = 2, kModeShadow = 3, kModeBa
 // more than J3DG_MAX_OBJECTS objects, with a top-level BVH over the objects
 // (FrameParams::top_nodes) and the object table read from global memory.
 constexpr int kModeTop = 16;
+// Added to kModeRays or kModeAnyRays on 8-wide trees: 2 to J3DG_MAX_OBJECTS objects.
+constexpr int kModeMany = 8;
 // Largest object count of one scene with a top level.
 constexpr uint32_t kMaxSceneObjects = 1u << 16;
 
