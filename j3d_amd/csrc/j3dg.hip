@@ -1472,6 +1472,34 @@ int Ctx::ensure_shadow_queue(uint64_t rays) {
   return J3DG_OK;
 }
 
+// The cost order pays from ~8192 tiles up: at 640x480 (4800 tiles) its three
+// sorting launches cost 20 us more than they save, at 1280x720 (14400) they save 24 us.
+bool Ctx::cost_ordered(const FrameParams& fp, const Target* tg) const {
+  return tg && tuning.cost_order && fp.n_obj && fp.n_tiles >= kOrderMinTiles;
+}
+
+// The target's buffers of a frame in cost order.  Learned frames call it before
+// the network's start event: the stage ends at the trace's start, and a first
+// frame's allocations are no part of it.
+int Ctx::ensure_tile_order(const FrameParams& fp, Target* tg) {
+  Ctx* ctx = this;
+  if (!cost_ordered(fp, tg) || fp.n_tiles <= tg->order_capacity) return J3DG_OK;
+  HIP_TRY(hipStreamSynchronize(stream), J3DG_ERR_LAUNCH);
+  if (tg->pixel_cost) hipFree(tg->pixel_cost);
+  if (tg->tile_cost) hipFree(tg->tile_cost);
+  if (tg->tile_order) hipFree(tg->tile_order);
+  tg->pixel_cost = nullptr, tg->tile_cost = nullptr, tg->tile_order = nullptr;
+  tg->order_capacity = 0;
+  tg->order_valid = false;
+  HIP_TRY(hipMalloc(&tg->pixel_cost, (size_t)fp.n_tiles * 64 * sizeof(uint16_t)), J3DG_ERR_OUT_OF_MEMORY);
+  const size_t nb = (fp.n_tiles + kOrderBlock - 1) / kOrderBlock;
+  HIP_TRY(hipMalloc(&tg->tile_cost, ((fp.n_tiles + 3) / 4 + nb * kOrderBins) * sizeof(uint32_t)),
+          J3DG_ERR_OUT_OF_MEMORY);
+  HIP_TRY(hipMalloc(&tg->tile_order, (size_t)fp.n_tiles * sizeof(uint32_t)), J3DG_ERR_OUT_OF_MEMORY);
+  tg->order_capacity = fp.n_tiles;
+  return J3DG_OK;
+}
+
 // The trace stage.  Fused (default): one k_trace launch whose lanes complete
 // their hits and trace the shadow rays.  Split: primary trace, k_finish
 // (normals, db_id, shadow queue) and the shadow trace.
@@ -1486,25 +1514,10 @@ int Ctx::launch_trace(const FrameParams& fp_in, uint32_t max_stack, int width, b
   const int top = fp.top_nodes ? kModeTop : 0;
   fp.fused = ((tuning.split_passes == 0 || top) && fp.n_obj) ? 1u : 0u;
   const uint32_t rect_px = fp.n_tiles * 64u;
-  // the cost order pays from ~8192 tiles up: at 640x480 (4800 tiles) its three
-  // sorting launches cost 20 us more than they save, at 1280x720 (14400) they save 24 us
-  const bool order = tg && tuning.cost_order && fp.n_obj && fp.n_tiles >= kOrderMinTiles;
+  int rc = ensure_tile_order(fp, tg);
+  if (rc) return rc;
+  const bool order = cost_ordered(fp, tg);
   if (order) {
-    if (fp.n_tiles > tg->order_capacity) {
-      HIP_TRY(hipStreamSynchronize(stream), J3DG_ERR_LAUNCH);
-      if (tg->pixel_cost) hipFree(tg->pixel_cost);
-      if (tg->tile_cost) hipFree(tg->tile_cost);
-      if (tg->tile_order) hipFree(tg->tile_order);
-      tg->pixel_cost = nullptr, tg->tile_cost = nullptr, tg->tile_order = nullptr;
-      tg->order_capacity = 0;
-      tg->order_valid = false;
-      HIP_TRY(hipMalloc(&tg->pixel_cost, (size_t)fp.n_tiles * 64 * sizeof(uint16_t)), J3DG_ERR_OUT_OF_MEMORY);
-      const size_t nb = (fp.n_tiles + kOrderBlock - 1) / kOrderBlock;
-      HIP_TRY(hipMalloc(&tg->tile_cost, ((fp.n_tiles + 3) / 4 + nb * kOrderBins) * sizeof(uint32_t)),
-              J3DG_ERR_OUT_OF_MEMORY);
-      HIP_TRY(hipMalloc(&tg->tile_order, (size_t)fp.n_tiles * sizeof(uint32_t)), J3DG_ERR_OUT_OF_MEMORY);
-      tg->order_capacity = fp.n_tiles;
-    }
     const bool same = tg->order_valid && tg->order_rect[0] == fp.x0 && tg->order_rect[1] == fp.y0 &&
                       tg->order_rect[2] == fp.x1 && tg->order_rect[3] == fp.y1;
     fp.tile_order = same ? tg->tile_order : nullptr;
@@ -1522,8 +1535,8 @@ int Ctx::launch_trace(const FrameParams& fp_in, uint32_t max_stack, int width, b
     return J3DG_OK;
   }
   const bool color = fp.fused && (fp.flags & (J3DG_TEXTURED | J3DG_VERTEXCOLORS));
-  int rc = launch_trace_kernel((color ? kModeFrameColor : kModeFrame) | top, fp, q, rect_px, fp.n_obj, max_stack,
-                               width, d_queue);
+  rc = launch_trace_kernel((color ? kModeFrameColor : kModeFrame) | top, fp, q, rect_px, fp.n_obj, max_stack, width,
+                           d_queue);
   if (rc) return rc;
   if (color) {
     const uint32_t n = (uint32_t)std::min<uint64_t>(((uint64_t)fp.n_tiles * 64 + 255) / 256, (uint64_t)n_cus * 16);
@@ -2328,6 +2341,8 @@ int j3dg_render(j3dg_ctx* h, const j3dg_frame_desc* fd, uint32_t target, uint32_
           if (rc) return rc;
           fp.proposal = tg.proposal;
           if (!keep) {
+            rc = ctx->ensure_tile_order(fp, &tg);
+            if (rc) return rc;
             rc = ctx->launch_mlp_frame(fp, fp.n_obj);
             if (rc) return rc;
           }

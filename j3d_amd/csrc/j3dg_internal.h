@@ -311,6 +311,8 @@ struct Ctx {
   int launch_mlp_frame(const FrameParams& fp, uint32_t n_obj, const DevObject* objs = nullptr, bool first = true,
                        bool last = true);
   int reset_counters();  // work-queue heads and statistics counters, for a launch that follows
+  bool cost_ordered(const FrameParams& fp, const Target* tg) const;
+  int ensure_tile_order(const FrameParams& fp, Target* tg);
   int launch_trace(const FrameParams& fp, uint32_t max_stack, int width, bool learned, Target* tg = nullptr);
   int launch_trace_kernel(int mode, const FrameParams& fp, const RayQuery& q, uint32_t n_rays, uint32_t n_obj,
                           uint32_t max_stack, int width, uint32_t* qcounter, const BatchParams* bp = nullptr);
