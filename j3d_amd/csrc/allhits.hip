@@ -205,11 +205,18 @@ __device__ inline void write_voxel(const AllHitsArgs& a, const HitRec& h, uint32
 // The voxel rays of all three axes.  A ray along an axis crosses the whole
 // mesh, hundreds of dependent node fetches where it grazes the surface, and a
 // grid has few of them (256 x 224 x 128: 118,000, two waves per SIMD with one
-// ray per lane, each as long as its longest ray: 714 us).  So a group of
+// ray per lane, each as long as its longest ray).  So a group of
 // kVoxLanes lanes takes a ray: each walks its own part of the tree, and idle
 // lanes take entries from the others' stacks after every step.  Order does not
 // matter here, so nodes are not sorted.  Waves take rounds of 64 / kVoxLanes
-// rays, a round's lists being the waves' own.
+// rays, a round's lists being the waves' own.  One lane / eight lanes per ray, us:
+//   2M triangles      256 per side  605 /  121   512   826 /  340   1024 1935 / 1144
+//   28M triangles                  1032 /  187        1294 /  508        3081 / 1530
+//   100,000 triangles               376 /   77         512 /  249        1135 /  873
+//   20,000, a dense soup            812 /  347        2094 / 1211
+//   1,280 triangles                  97 /   82         265 /  292         790 / 1131
+// Only a coarse mesh on a large grid has rays too short to share; its call
+// (13.5 and 105 ms) is the grid's copy to the host.
 constexpr uint32_t kVoxLanes = 8;
 constexpr uint32_t kVoxGroups = kAllBlock / kVoxLanes;
 // Hits of a ray ranked by counting (k^2 / 8 reads per lane); more are sorted.
@@ -377,8 +384,8 @@ int launch_all_hits(Ctx* ctx, const Mesh& m, AllHitsArgs& a, uint32_t grid, bool
   return J3DG_OK;
 }
 
-// Blocks of a voxel launch: those the GPU holds at once (five by LDS, four
-// asked for by the kernel's register bound), or fewer for few rays.
+// Blocks of a voxel launch: those the GPU holds at once (four per CU, by the
+// kernel's register bound and by LDS: 32,896 bytes a block), or fewer for few rays.
 uint32_t vox_grid(uint32_t n, int n_cus) {
   return std::max(1u, std::min((n + kVoxGroups - 1) / kVoxGroups, (uint32_t)n_cus * 4u));
 }

@@ -45,7 +45,7 @@ constexpr int kStepsPerTrip = 4;
 // Scenes with a top level: a lane done with an object waits for the next walk
 // of the top level, one per kTopWalk steps for all such lanes.  A walk after
 // every step, for whichever lanes need one, ran the walk's code with a few
-// lanes each time (256 objects, 1080p, frames one at a time: 1.43 ms; one walk
+// lanes each time (256 objects, 1366x767, frames one at a time: 1.43 ms; one walk
 // every 5 steps and the split tail below: 0.94 ms; every 3, 4 and, with one
 // walk per trip, 8 steps: 0.95, 0.94, 1.03 ms).
 constexpr int kTopWalk = 5;
@@ -782,7 +782,7 @@ __global__ void __launch_bounds__(256) k_color(FrameParams f, const DevObject* _
 // rectangle gets the miss fields; mark, r, g, b and the barycentrics keep their
 // values.  One word per thread, so that a wave's store covers 64 consecutive
 // words (five of every eight are written): bound by the 64 MB of lines a 1080p
-// G-buffer holds.  (As rays through k_trace: 163-174 us; so: 21 us.)
+// G-buffer holds.  (As rays through k_trace: 163-174 us; so: 24 us.)
 __global__ void __launch_bounds__(256) k_miss(FrameParams f, uint64_t* counters) {
   const uint32_t n_words = f.x1 >= f.x0 ? (uint32_t)(f.x1 - f.x0 + 1) * 8u : 0u;
   const uint32_t k = threadIdx.x & 7u;  // word of the pixel; 1, 2: normal, 3: depth, 4: object_id, 7: db_id
@@ -947,7 +947,9 @@ constexpr uint32_t kOrderMinTiles = 8192;  // smallest rectangle (in 8x8 tiles) 
 // A tile holding a pixel of at least this many loop trips goes to the heaviest
 // bin whatever its sum, so that the frame's longest pixels start first (28M-
 // triangle 1080p frame: 0.784-0.789 ms without; threshold 24: 0.93, 32: 0.83,
-// 40: 0.753-0.778, 48: 0.761, 64: 0.777)
+// 40: 0.753-0.778, 48: 0.761, 64: 0.777).  Scenes with a top level, whose trips are
+// of up to kTopSteps steps and waits: 12, 24, 48 and no threshold differ by at most
+// 1 % (17 to 3000 objects, 1366x767 and 1080p).
 constexpr uint32_t kLongPixelTrips = 48;
 
 __device__ inline uint32_t cost_bin(uint32_t c) {
@@ -2745,7 +2747,7 @@ int j3dg_render_batch(j3dg_ctx* h, const j3dg_frame_desc* frames, const uint32_t
   // the learned frames' proposals, before the graph (they change with the cameras)
   for (size_t k = 0; k < infer.size(); ++k) {
     const uint32_t i = infer[k];
-    rc = ctx->launch_mlp_frame(fps[i], fps[i].n_obj, ctx->d_bobjs + fps[i].obj_base, k == 0, k + 1 == infer.size());
+    rc = ctx->launch_mlp_frame(fps[i], fps[i].n_obj, ctx->d_bobjs + fps[i].obj_base, k == 0);
     if (rc) return rc;
   }
   hipEvent_t* e = ctx->cur_ev();

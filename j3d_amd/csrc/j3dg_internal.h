@@ -306,8 +306,8 @@ struct Ctx {
   // learned proposal for the frame's objects into fp.proposal (mlp.hip)
   // the proposal network over a frame's pixels into fp.proposal; objs: the frame's
   // object table (nullptr: the current single-frame table); the render's mlp
-  // start event is recorded before the launch when `first`; after the `last` one
-  // the trace's start event, which follows, is the stage's end
+  // start event is recorded before the launch when `first`; the stage ends at the
+  // trace's start event, which follows the last one (nothing reads the `last` argument)
   int launch_mlp_frame(const FrameParams& fp, uint32_t n_obj, const DevObject* objs = nullptr, bool first = true,
                        bool last = true);
   int reset_counters();  // work-queue heads and statistics counters, for a launch that follows
