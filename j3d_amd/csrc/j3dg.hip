@@ -803,7 +803,7 @@ constexpr uint32_t kCounters = 32;
 __global__ void k_reset(uint32_t* queue, uint64_t* counters, uint32_t n_counters) {
   uint32_t i = threadIdx.x;
   for (uint32_t k = i; k < kQueueWords; k += blockDim.x) queue[k] = 0u;
-  for (uint32_t k = i; k < n_counters; k += blockDim.x) counters[k] = 0ull;
+  if (i < n_counters) counters[i] = 0ull;
 }
 
 // canvas::canvas_to_image (j3d/canvas.cpp:582-670) with the background copy of
@@ -1779,9 +1779,10 @@ int j3dg_create(int device, j3dg_ctx** out) {
     if (hipEventCreate(&e) != hipSuccess) return cleanup(J3DG_ERR_LAUNCH);
   if (hipMalloc(&ctx->d_queue, kQueueWords * sizeof(uint32_t)) != hipSuccess) return cleanup(J3DG_ERR_OUT_OF_MEMORY);
   if (hipMalloc(&ctx->d_counters, 2 * kCounters * sizeof(uint64_t)) != hipSuccess) return cleanup(J3DG_ERR_OUT_OF_MEMORY);
-  // no counts before the first render, whatever the memory held
-  hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, ctx->stream, ctx->d_queue, ctx->d_counters, 2 * kCounters);
-  if (hipGetLastError() != hipSuccess) return cleanup(J3DG_ERR_LAUNCH);
+  // no counts before the first render, whatever the memory held (the call's own status: an error
+  // that an earlier call on this thread left behind is none of this context's)
+  if (hipMemsetAsync(ctx->d_counters, 0, 2 * kCounters * sizeof(uint64_t), ctx->stream) != hipSuccess)
+    return cleanup(J3DG_ERR_LAUNCH);
   if (noalloc_scratch_setup(device, &ctx->noalloc_scratch) != J3DG_OK) return cleanup(J3DG_ERR_LAUNCH);
   *out = reinterpret_cast<j3dg_ctx*>(ctx);
   return J3DG_OK;

@@ -1,5 +1,8 @@
 """A context that has rendered nothing has no counts, whatever the memory that
-it was given held before."""
+it was given held before, and an error that some other call left behind on the
+thread does not keep it from being made."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -27,3 +30,13 @@ def test_counters_start_at_zero():
         with J.Renderer(0) as r:
             counts = {k: x for k, x in r.stats().items() if not k.endswith("_ms")}
             assert all(not np.any(x) for x in counts.values()), (n, counts)
+
+
+def test_an_error_left_behind_by_another_call():
+    hip = ctypes.CDLL("libamdhip64.so")
+    assert hip.hipSetDevice(9999) != 0 and hip.hipPeekAtLastError() != 0
+    try:
+        with J.Renderer(0) as r:
+            assert r.stats()["primary_rays"] == 0
+    finally:
+        hip.hipGetLastError()  # clears it
